@@ -15,7 +15,7 @@ import torch  # noqa: F401  (must precede CDLL, see module docstring)
 
 MAX_PATHS = 128
 LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "lib", "libictc_hip.so")
-ABI_VERSION = 21
+ABI_VERSION = 22
 
 
 class TpDesc(ctypes.Structure):
@@ -111,6 +111,10 @@ _SIGNATURES = {
     "ictc_hip_radial_mlp_workspace": (_I64, [_I64]),
     "ictc_hip_radial_mlp": (ctypes.c_int, [ctypes.c_int, _P, _P, _P, _P, ctypes.c_float, _P, _P, _P, _P, _P, _P, _I64,
                                            _P, _P, _P, ctypes.c_int, _I64, _P]),
+    "ictc_hip_gates_forward": (ctypes.c_int, [_P, _P, _I64, _I64, _P, _I64, _I64, _I64, _P]),
+    "ictc_hip_gates_input_grad": (ctypes.c_int, [_P, _I64, _P, _I64, _I64, _P, _I64, _I64, _P]),
+    "ictc_hip_gates_weight_grad_workspace": (_I64, [_I64, _I64]),
+    "ictc_hip_gates_weight_grad": (ctypes.c_int, [_P, _I64, _P, _P, _I64, _P, _I64, _I64, _I64, _I64, _P]),
     "ictc_hip_sgemm": (ctypes.c_int, [ctypes.c_int, ctypes.c_int, _I64, _I64, _I64, ctypes.c_float, _P, _I64, _P,
                                       _I64, ctypes.c_float, _P, _I64, _P]),
     "ictc_hip_radius_graph_count": (ctypes.c_int, [ctypes.POINTER(CellGrid), _P, _P, _P, _P, _I64, _P, _P]),

@@ -1,0 +1,107 @@
+"""Products with a 64-wide inner side over edge-sized rows on ``ictc_hip_gates_*`` (fp32 operands in
+three bf16 parts on the matrix cores): the radial network's last layer ``h W^T`` (reference
+``mace_ictc/models/pure_cartesian_ictd_fix.py:1545-1553``), its input adjoint ``g W`` and its
+weight adjoint ``g^T h``.  ``product`` recognises the three forms in ``a @ b``; ``linear.mm`` asks
+it first and keeps its library routes for every other shape.
+
+The lines between the routes (MI355X, us per call with its launches, the library's time in brackets):
+
+* forward from 2,048 rows: 10 (13) at 2,048 x 2,944, 25 (34) at 8,192 x 2,944, 275 (385) at 105,634 x
+  2,944, 38 (57) at 105,634 x 352; below, both are the launch;
+* input adjoint from 50,000 rows: a block takes 128 rows and a fixed 1.1 us per 32 columns, so fewer
+  rows leave CUs idle: 116 (106) at 32,768 x 2,944, 169 (220) at 50,000 x 2,944, 300 (353) at 105,634 x
+  2,944, 48 (54) at 50,000 x 704;
+* weight adjoint from 2,048 rows: 24 (68) at 2,048 x 2,944, 18 (28) at 8,192 x 352, 287 (620) at 105,634 x
+  2,944; up to 4,096 rows and 704 columns the two are within 3 us of each other.
+"""
+from __future__ import annotations
+
+from typing import Optional
+
+import torch
+
+from ... import _lib
+
+WIDTH = 64
+MIN_OUTER = 128            # narrower outer sides stay on the library (its 64 x 64 products take one tile)
+FORWARD_ROWS = 2048
+INPUT_GRAD_ROWS = 50000
+WEIGHT_GRAD_ROWS = 2048
+MAX_OUTER = 1 << 20
+MAX_ROW_STRIDE = 1 << 22
+
+
+def _rows(t: torch.Tensor, width: int) -> bool:
+    """t [R, width] read row by row: unit column stride, rows that do not overlap."""
+    return t.stride(1) == 1 and width <= t.stride(0) <= MAX_ROW_STRIDE
+
+
+def _hidden(t: torch.Tensor) -> bool:
+    return t.stride(1) == 1 and t.stride(0) == WIDTH and t.data_ptr() % 16 == 0
+
+
+def _weight(t: torch.Tensor) -> bool:
+    """t [outer, 64] within the kernels' 32-bit byte offsets."""
+    sn, sk = t.stride()
+    return 0 <= sn <= 1 << 28 and 0 <= sk <= 1 << 22 and (t.shape[0] - 1) * sn + (WIDTH - 1) * sk < 1 << 29
+
+
+def _forward(hidden: torch.Tensor, weight: torch.Tensor, out: Optional[torch.Tensor]) -> torch.Tensor:
+    edges, width = hidden.shape[0], weight.shape[0]
+    if out is None:
+        out = torch.empty(edges, width, device=hidden.device, dtype=torch.float32)
+    _lib.check(_lib.lib().ictc_hip_gates_forward(
+        hidden.data_ptr(), weight.data_ptr(), weight.stride(0), weight.stride(1), out.data_ptr(), out.stride(0), edges,
+        width, _lib.stream_of(hidden.device)), "ictc_hip_gates_forward")
+    return out
+
+
+def _input_grad(grad: torch.Tensor, weight: torch.Tensor, out: Optional[torch.Tensor]) -> torch.Tensor:
+    edges, width = grad.shape
+    if out is None:
+        out = torch.empty(edges, WIDTH, device=grad.device, dtype=torch.float32)
+    _lib.check(_lib.lib().ictc_hip_gates_input_grad(
+        grad.data_ptr(), grad.stride(0), weight.data_ptr(), weight.stride(0), weight.stride(1), out.data_ptr(), edges,
+        width, _lib.stream_of(grad.device)), "ictc_hip_gates_input_grad")
+    return out
+
+
+def _weight_grad(grad: torch.Tensor, hidden: torch.Tensor, transposed: bool) -> torch.Tensor:
+    """g^T h [N, 64], or its transpose [64, N]."""
+    edges, width = grad.shape
+    lib, dev = _lib.lib(), grad.device
+    floats = int(lib.ictc_hip_gates_weight_grad_workspace(edges, width))
+    if floats < 0:
+        _lib.check(-floats, "ictc_hip_gates_weight_grad_workspace")
+    ws = torch.empty(max(floats, 1), device=dev, dtype=torch.float32)
+    out = torch.empty((WIDTH, width) if transposed else (width, WIDTH), device=dev, dtype=torch.float32)
+    strides = (1, width) if transposed else (WIDTH, 1)
+    _lib.check(lib.ictc_hip_gates_weight_grad(
+        grad.data_ptr(), grad.stride(0), hidden.data_ptr(), ws.data_ptr(), floats, out.data_ptr(), *strides, edges,
+        width, _lib.stream_of(dev)), "ictc_hip_gates_weight_grad")
+    return out
+
+
+def product(a: torch.Tensor, b: torch.Tensor, out: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
+    """a [M, K] @ b [K, N] when it is one of the three forms at a size they are the faster route
+    for; None otherwise.  out: a caller's row-major result (the first two forms; a row slice of a
+    wider matrix for the first)."""
+    if not a.is_cuda or a.dtype != torch.float32 or b.dtype != torch.float32 or a.device != b.device:
+        return None
+    m, k = a.shape
+    n = b.shape[1]
+    if k == WIDTH:
+        if (FORWARD_ROWS <= m and MIN_OUTER <= n <= MAX_OUTER and _hidden(a) and _weight(b.t())
+                and (out is None or _rows(out, n))):
+            return _forward(a, b.t(), out)
+        return None
+    if (n == WIDTH and m >= INPUT_GRAD_ROWS and MIN_OUTER <= k <= MAX_OUTER and k % 4 == 0 and _rows(a, k)
+            and a.stride(0) % 4 == 0 and a.data_ptr() % 16 == 0 and _weight(b)
+            and (out is None or (out.stride(0) == WIDTH and out.stride(1) == 1))):
+        return _input_grad(a, b, out)
+    if k >= WEIGHT_GRAD_ROWS and out is None:
+        if n == WIDTH and MIN_OUTER <= m <= MAX_OUTER and _rows(a.t(), m) and b.stride(1) == 1 and b.stride(0) == WIDTH:
+            return _weight_grad(a.t(), b, False)
+        if m == WIDTH and MIN_OUTER <= n <= MAX_OUTER and _rows(b, n) and a.stride(0) == 1 and a.stride(1) == WIDTH:
+            return _weight_grad(b, a.t(), True)
+    return None

@@ -8,12 +8,13 @@ not run skipped.
 
 Routing of ``mm`` (measured on MI355X at the MACE cfg-4 shapes, E = 105,634 edges):
 
-* plain products call rocBLAS explicitly through ``ictc_hip_sgemm`` with the operands' own
+* edge-sized products with a 64-wide inner side (the gates, their input and weight adjoints) run on
+  the split-bf16 matrix-core kernels of ``gates``, which holds the sizes and times of that route;
+* other plain products call rocBLAS explicitly through ``ictc_hip_sgemm`` with the operands' own
   storage order passed as transpose flags (no copies, no process-wide library preference);
   an edge-sized left operand against a weight (``x @ W^T``, and ``g @ W`` in the backward, where
-  the weight-sized right operand is copied column-major) runs with a column-major right operand:
-  0.485 vs 0.571 ms for ``[E,64]@[64,2944]`` on hipBLASLt, 0.372 vs 0.39-0.41 ms for
-  ``[E,2944]@[2944,64]``; a short reduction (K < 16, ``[E,8]@[8,64]``) keeps a row-major right
+  the weight-sized right operand is copied column-major) runs with a column-major right operand,
+  rocBLAS's faster layout; a short reduction (K < 16, ``[E,8]@[8,64]``) keeps a row-major right
   operand (25 vs 35 us);
 * a weight gradient ``g^T x`` reduces over ~10^5 rows into a small output, which one GEMM
   covers with a handful of output tiles (0.3 ms for 0.9 GFLOP); it is split into row blocks
@@ -26,6 +27,7 @@ import torch
 
 from ... import _lib
 from ...autograd.adjoint_requirements import required_gradients
+from . import gates
 from .runtime import require_gpu_fp32
 from .species import validate_species
 
@@ -72,7 +74,7 @@ def _sgemm(a: torch.Tensor, b: torch.Tensor, *, row_major_b: bool = False) -> to
 
 
 def sgemm_into(a: torch.Tensor, b: torch.Tensor, out: torch.Tensor) -> torch.Tensor:
-    """out = a [M, K] @ b [K, N] on rocBLAS with no autograd record, into a caller-owned row-major
+    """out = a [M, K] @ b [K, N] (a product of ``gates``, else rocBLAS) with no autograd record, into a caller-owned row-major
     out (a row slice of a larger matrix is fine); the operands' storage orders are passed as is."""
     m, k = a.shape
     n = b.shape[1]
@@ -82,6 +84,8 @@ def sgemm_into(a: torch.Tensor, b: torch.Tensor, out: torch.Tensor) -> torch.Ten
         return out
     if k == 0:
         return out.zero_()
+    if gates.product(a, b, out) is not None:
+        return out
     a, ta, lda = _storage(a)
     b, tb, ldb = _storage(b)
     _lib.check(_lib.lib().ictc_hip_sgemm(ta, tb, m, n, k, 1.0, a.data_ptr(), lda, b.data_ptr(), ldb, 0.0,
@@ -102,6 +106,9 @@ def _plain(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
 
 
 def _product(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
+    special = gates.product(a, b)
+    if special is not None:
+        return special
     m, k = a.shape
     n = b.shape[1]
     rows = SPLIT_ROWS_LARGE if m * n >= SPLIT_LARGE_OUTPUT else SPLIT_ROWS

@@ -620,6 +620,29 @@ int ictc_hip_degree_linear_weight_grad(const ictc_degree_linear_desc* desc, int 
                                        float* const* grad_weights, int64_t nodes, hipStream_t stream);
 
 /*
+ * Products with a 64-wide inner side (the radial network's last layer and its adjoints; reference
+ * mace_ictc/models/pure_cartesian_ictd_fix.py:1545-1553), fp32 operands in three bf16 parts on the
+ * matrix cores.  hidden [edges, 64] contiguous and 16-byte aligned; weight element (n, c) at
+ * n * weight_row_stride + c * weight_col_stride, n < width, c < 64:
+ *   forward      out[e, n]  = sum_c hidden[e, c] weight[n, c]      rows of out_row_stride floats
+ *   input_grad   out[e, c]  = sum_n grad[e, n] weight[n, c]        grad 16-byte aligned, its row
+ *                             stride and width multiples of 4 (else ICTC_ERR_UNSUPPORTED); out [edges, 64]
+ *   weight_grad  out(n, c)  = sum_e grad[e, n] hidden[e, c]        at n * out_row_stride + c *
+ *                             out_col_stride; workspace: _workspace() floats (negative: -ictc_status)
+ * Sums run in a fixed order.
+ */
+int ictc_hip_gates_forward(const float *hidden, const float *weight, int64_t weight_row_stride,
+                           int64_t weight_col_stride, float *out, int64_t out_row_stride, int64_t edges,
+                           int64_t width, hipStream_t stream);
+int ictc_hip_gates_input_grad(const float *grad, int64_t grad_row_stride, const float *weight,
+                              int64_t weight_row_stride, int64_t weight_col_stride, float *out, int64_t edges,
+                              int64_t width, hipStream_t stream);
+int64_t ictc_hip_gates_weight_grad_workspace(int64_t edges, int64_t width);
+int ictc_hip_gates_weight_grad(const float *grad, int64_t grad_row_stride, const float *hidden, float *workspace,
+                               int64_t workspace_floats, float *out, int64_t out_row_stride, int64_t out_col_stride,
+                               int64_t edges, int64_t width, hipStream_t stream);
+
+/*
  * Row-major fp32 product C[m,n] = alpha * op(A) op(B) + beta * C on rocBLAS, for the dense
  * channel linears around the operators.  op(A) is [m,k]: A is stored [m,k] (lda >= k) or,
  * with trans_a != 0, [k,m] (lda >= m); likewise B with op(B) [k,n].  Each host thread uses

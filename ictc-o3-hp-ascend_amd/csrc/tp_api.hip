@@ -8,10 +8,11 @@ namespace ictc {
 // Explicit instantiations live in separate translation units (parallel build).
 #define ICTC_DECLARE(A, B, C)                                                                  \
   extern template int launch_forward<A, B, C>(const ictc_tp_desc&, const float*, const float*,   \
-                                              const float*, float*, int64_t, hipStream_t);      \
+                                              const float*, const float*, float*, int64_t,      \
+                                              hipStream_t);                                     \
   extern template int launch_backward<A, B, C>(const ictc_tp_desc&, const float*, const float*,  \
-                                               const float*, const float*, float*, float*, float*, \
-                                               int64_t, hipStream_t);
+                                               const float*, const float*, const float*, float*,   \
+                                               float*, float*, int64_t, hipStream_t);
 #include "generated/tp_instances.def"
 #undef ICTC_DECLARE
 
@@ -19,10 +20,11 @@ namespace ictc {
 // degree-generic kernels.
 #define ICTC_DECLARE(A, B, C)                                                                  \
   extern template int launch_forward<A, B, C>(const ictc_tp_desc&, const float*, const float*,   \
-                                              const float*, float*, int64_t, hipStream_t);      \
+                                              const float*, const float*, float*, int64_t,      \
+                                              hipStream_t);                                     \
   extern template int launch_backward<A, B, C>(const ictc_tp_desc&, const float*, const float*,  \
-                                               const float*, const float*, float*, float*, float*, \
-                                               int64_t, hipStream_t);
+                                               const float*, const float*, const float*, float*,   \
+                                               float*, float*, int64_t, hipStream_t);
 #include "generated/tp_wide_instances.def"
 #undef ICTC_DECLARE
 
@@ -97,7 +99,7 @@ const char* ictc_hip_status_string(int status) {
   }
 }
 
-int ictc_hip_abi_version(void) { return 22; }
+int ictc_hip_abi_version(void) { return 23; }
 
 int ictc_hip_tp_slot_count(int input_lmax, int edge_lmax, int output_lmax) {
   constexpr int L = ictc::kGenericMaxL;
@@ -106,25 +108,43 @@ int ictc_hip_tp_slot_count(int input_lmax, int edge_lmax, int output_lmax) {
   return ictc::make_paths(input_lmax, edge_lmax, output_lmax).n;
 }
 
-int ictc_hip_tp_forward(const ictc_tp_desc* desc, const float* features, const float* harmonics,
-                        const float* gates, float* out, int64_t rows, hipStream_t stream) {
+// Widest path weight [P, C] (floats) the degree set's kernels fold into the gates: 0 for the sets of
+// the run-time-table kernels.
+int ictc_hip_tp_weight_capacity(const ictc_tp_desc* desc) {
+  if (ictc::tp_check_desc(desc) != ICTC_OK) return -1;
+  if (ictc::wide_forward(desc) != nullptr) return ictc::kTpWeightMax;
+  if (ictc::generic_degrees(*desc)) return 0;
+  return ictc::kFwdTable[ictc::table_index(desc)] != nullptr ? ictc::kTpWeightMax : 0;
+}
+
+int ictc_hip_tp_forward_weighted(const ictc_tp_desc* desc, const float* features, const float* harmonics,
+                                 const float* gates, const float* path_weight, float* out, int64_t rows,
+                                 hipStream_t stream) {
   const int st = ictc::tp_check_desc(desc);
   if (st != ICTC_OK) return st;
   if (rows < 0) return ICTC_ERR_INVALID_ARGUMENT;
   if (rows == 0) return ICTC_OK;
   if (!features || !harmonics || !gates || !out) return ICTC_ERR_INVALID_ARGUMENT;
+  if (path_weight && int64_t{desc->num_paths} * desc->channels > ictc_hip_tp_weight_capacity(desc))
+    return ICTC_ERR_UNSUPPORTED;
   if (const ictc::FwdLaunch wide = ictc::wide_forward(desc))
-    return wide(*desc, features, harmonics, gates, out, rows, stream);
+    return wide(*desc, features, harmonics, gates, path_weight, out, rows, stream);
   if (ictc::generic_degrees(*desc))
     return ictc::generic_tp_forward(*desc, features, harmonics, gates, out, rows, stream);
   const ictc::FwdLaunch fn = ictc::kFwdTable[ictc::table_index(desc)];
   if (fn == nullptr) return ICTC_ERR_UNSUPPORTED;
-  return fn(*desc, features, harmonics, gates, out, rows, stream);
+  return fn(*desc, features, harmonics, gates, path_weight, out, rows, stream);
 }
 
-int ictc_hip_tp_backward(const ictc_tp_desc* desc, const float* features, const float* harmonics,
-                         const float* gates, const float* grad_out, float* grad_features,
-                         float* grad_harmonics, float* grad_gates, int64_t rows, hipStream_t stream) {
+int ictc_hip_tp_forward(const ictc_tp_desc* desc, const float* features, const float* harmonics,
+                        const float* gates, float* out, int64_t rows, hipStream_t stream) {
+  return ictc_hip_tp_forward_weighted(desc, features, harmonics, gates, nullptr, out, rows, stream);
+}
+
+int ictc_hip_tp_backward_weighted(const ictc_tp_desc* desc, const float* features, const float* harmonics,
+                                  const float* gates, const float* path_weight, const float* grad_out,
+                                  float* grad_features, float* grad_harmonics, float* grad_gates, int64_t rows,
+                                  hipStream_t stream) {
   const int st = ictc::tp_check_desc(desc);
   if (st != ICTC_OK) return st;
   if (rows < 0) return ICTC_ERR_INVALID_ARGUMENT;
@@ -132,16 +152,25 @@ int ictc_hip_tp_backward(const ictc_tp_desc* desc, const float* features, const 
   if (!harmonics || !gates || !grad_out) return ICTC_ERR_INVALID_ARGUMENT;
   if ((grad_harmonics || grad_gates) && !features) return ICTC_ERR_INVALID_ARGUMENT;
   if (!grad_features && !grad_harmonics && !grad_gates) return ICTC_OK;
+  if (path_weight && int64_t{desc->num_paths} * desc->channels > ictc_hip_tp_weight_capacity(desc))
+    return ICTC_ERR_UNSUPPORTED;
   if (const ictc::BwdLaunch wide = ictc::wide_backward(desc))
-    return wide(*desc, features, harmonics, gates, grad_out, grad_features, grad_harmonics, grad_gates, rows,
-                stream);
+    return wide(*desc, features, harmonics, gates, path_weight, grad_out, grad_features, grad_harmonics, grad_gates,
+                rows, stream);
   if (ictc::generic_degrees(*desc))
     return ictc::generic_tp_backward(*desc, features, harmonics, gates, grad_out, grad_features, grad_harmonics,
                                      grad_gates, rows, stream);
   const ictc::BwdLaunch fn = ictc::kBwdTable[ictc::table_index(desc)];
   if (fn == nullptr) return ICTC_ERR_UNSUPPORTED;
-  return fn(*desc, features, harmonics, gates, grad_out, grad_features, grad_harmonics, grad_gates,
+  return fn(*desc, features, harmonics, gates, path_weight, grad_out, grad_features, grad_harmonics, grad_gates,
             rows, stream);
+}
+
+int ictc_hip_tp_backward(const ictc_tp_desc* desc, const float* features, const float* harmonics,
+                         const float* gates, const float* grad_out, float* grad_features,
+                         float* grad_harmonics, float* grad_gates, int64_t rows, hipStream_t stream) {
+  return ictc_hip_tp_backward_weighted(desc, features, harmonics, gates, nullptr, grad_out, grad_features,
+                                       grad_harmonics, grad_gates, rows, stream);
 }
 
 }  // extern "C"

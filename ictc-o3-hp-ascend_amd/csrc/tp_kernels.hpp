@@ -90,14 +90,36 @@ __device__ __forceinline__ void stage_tile(const float* __restrict__ y, int64_t 
   __syncthreads();
 }
 
+// Path weights.  A frozen per-(path, channel) weight [P, C] multiplies the gates inside the kernels
+// (out += (g w) x M; dg = w (g w)-gradient), each product rounded as in a separate g * w pass, so the
+// results are bit-identical to it: the passes over the [rows, P C] gates and gate gradients (2 x 0.48 ms
+// of 4.76 ms at C128/lmax3, 131,072 instances) go away.  A workgroup stages the weight in LDS once;
+// WEIGHTED = false kernels take gates that carry it already.
+constexpr int kTpWeightMax = 4096;   // P * C floats of LDS; wider products keep the separate pass
+
+template <bool WEIGHTED, int NT = kBlock>
+__device__ __forceinline__ void stage_weight(const float* __restrict__ w, float* sW, int n, int tid) {
+  if constexpr (WEIGHTED)
+    for (int t = tid; t < n; t += NT) sW[t] = w[t];   // (read after stage_tile's barriers)
+}
+
+template <bool WEIGHTED, int NV>
+__device__ __forceinline__ Vec<NV> path_weight(const float* sW, int at) {
+  Vec<NV> r;
+#pragma unroll
+  for (int v = 0; v < NV; ++v) r.v[v] = WEIGHTED ? sW[at + v] : 1.f;
+  return r;
+}
+
 // Forward.  Per instance the wave issues every feature and gate load up front
 // (NX + P row loads), then streams the NOC output rows; the path loop is fully
 // unrolled with compile-time output offsets, so the instance body is branch-free.
-template <int LIN, int LE, int LOUT, int NV>
+template <int LIN, int LE, int LOUT, int NV, bool WEIGHTED>
 __global__ void __launch_bounds__(kBlock)
 tp_forward_kernel(const float* __restrict__ x, const float* __restrict__ y,
-                  const float* __restrict__ g, float* __restrict__ out,
+                  const float* __restrict__ g, const float* __restrict__ w, float* __restrict__ out,
                   const ictc_tp_desc d, int64_t rows) {
+  extern __shared__ float sW[];   // WEIGHTED: [P, C]
   using PS = Paths<LIN, LE, LOUT>;
   constexpr int NX = PS::NX, NY = PS::NY, NP = PS::N, NOC = PS::NOC;
   constexpr int NBS = PS::NB > 0 ? PS::NB : 1;
@@ -121,6 +143,7 @@ tp_forward_kernel(const float* __restrict__ x, const float* __restrict__ y,
 #pragma unroll
   for (int m = 0; m < NX; ++m) xr0[m] = buf_load<NV>(rx0, vo0 + m * row);
 
+  stage_weight<WEIGHTED>(w, sW, NP * C, tid);
   stage_tile<LIN, LE, LOUT, kFwdTile>(y, e0, rows, sY, sM, d, tid);
 
   for (int le = wave; le < kFwdTile; le += kWavesPerBlock) {
@@ -148,6 +171,11 @@ tp_forward_kernel(const float* __restrict__ x, const float* __restrict__ y,
         constexpr int l1 = PS::tab.l1[p], l3 = PS::tab.l3[p];
         constexpr int ni = 2 * l1 + 1, no = 2 * l3 + 1;
         constexpr int boff = PS::tab.bond[p], oo = PS::tab.out[p];
+        if constexpr (WEIGHTED) {
+          const Vec<NV> wv = path_weight<true, NV>(sW, p * C + c);
+#pragma unroll
+          for (int v = 0; v < NV; ++v) gv[p].v[v] *= wv.v[v];
+        }
         static_for<0, no>([&](auto K) {
           Vec<NV> acc;
 #pragma unroll
@@ -180,12 +208,13 @@ tp_forward_kernel(const float* __restrict__ x, const float* __restrict__ y,
 // dropped by the hardware range check, so the instance body has no branches.
 // NV = 2 asks for three waves per SIMD (168 registers; the <3,3,3,2> instance needs 170 without
 // the bound and measured 2.07 ms at two waves per SIMD, 2.04 ms at three).
-template <int LIN, int LE, int LOUT, int NV>
+template <int LIN, int LE, int LOUT, int NV, bool WEIGHTED>
 __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(NV == 2 ? 3 : 1)))
 tp_backward_kernel(const float* __restrict__ x, const float* __restrict__ y,
-                   const float* __restrict__ g, const float* __restrict__ go,
+                   const float* __restrict__ g, const float* __restrict__ w, const float* __restrict__ go,
                    float* __restrict__ dx, float* __restrict__ dy, float* __restrict__ dg,
                    const ictc_tp_desc d, int64_t rows) {
+  extern __shared__ float sW[];   // WEIGHTED: [P, C]
   using PS = Paths<LIN, LE, LOUT>;
   constexpr int NX = PS::NX, NY = PS::NY, NP = PS::N, NOC = PS::NOC;
   constexpr int NBS = PS::NB > 0 ? PS::NB : 1;
@@ -206,6 +235,7 @@ tp_backward_kernel(const float* __restrict__ x, const float* __restrict__ y,
   Vec<NV> xr0[NX];
 #pragma unroll
   for (int m = 0; m < NX; ++m) xr0[m] = buf_load<NV, kNonTemporal>(rx0, vo0 + m * row);
+  stage_weight<WEIGHTED>(w, sW, NP * C, tid);
   stage_tile<LIN, LE, LOUT, kBwdTile>(y, e0, rows, sY, sM, d, tid);
 
   for (int le = wave; le < kBwdTile; le += kWavesPerBlock) {
@@ -254,7 +284,12 @@ tp_backward_kernel(const float* __restrict__ x, const float* __restrict__ y,
         constexpr int ni = 2 * l1 + 1, nj = 2 * l2 + 1, no = 2 * l3 + 1;
         constexpr int boff = PS::tab.bond[p];
         using CG = CGTab<l1, l2, l3>;
-        const Vec<NV> gv = pre_g[p % D];
+        const Vec<NV> wv = path_weight<WEIGHTED, NV>(sW, p * C + c);
+        Vec<NV> gv = pre_g[p % D];
+        if constexpr (WEIGHTED) {
+#pragma unroll
+          for (int v = 0; v < NV; ++v) gv.v[v] *= wv.v[v];
+        }
         Vec<NV> o[no];
         static_for<0, no>([&](auto K) { o[K] = pre_o[p % D][K]; });
         request(Int<p + D>{});             // issued ahead of this path's dg store
@@ -282,6 +317,10 @@ tp_backward_kernel(const float* __restrict__ x, const float* __restrict__ y,
 #pragma unroll
           for (int v = 0; v < NV; ++v) dgv.v[v] = fmaf(base.v[v], o[K].v[v], dgv.v[v]);
         });
+        if constexpr (WEIGHTED) {
+#pragma unroll
+          for (int v = 0; v < NV; ++v) dgv.v[v] *= wv.v[v];
+        }
         buf_store<NV>(rdg, vo + p * row, dgv);
         float part[nj];
 #pragma unroll
@@ -327,10 +366,11 @@ constexpr int first_path_of_degree(int a) {
 // wave per SIMD, 2.91 ms); 247 per degree (two waves, 1.89 ms); 118 with the single pass over
 // the bond entries (four waves, 1.44 ms); one-wave workgroups 1.415 ms.
 constexpr int kWideBlock = kWave;
-template <int LIN, int LE, int LOUT>
+// A path weight is requested with the path's gate row (a one-wave workgroup would stage it for one use).
+template <int LIN, int LE, int LOUT, bool WEIGHTED>
 __global__ void __launch_bounds__(kWideBlock)
 tp_backward_wide_kernel(const float* __restrict__ x, const float* __restrict__ y,
-                        const float* __restrict__ g, const float* __restrict__ go,
+                        const float* __restrict__ g, const float* __restrict__ w, const float* __restrict__ go,
                         float* __restrict__ dx, float* __restrict__ dy, float* __restrict__ dg,
                         const ictc_tp_desc d, int64_t rows) {
   using PS = Paths<LIN, LE, LOUT>;
@@ -351,6 +391,7 @@ tp_backward_wide_kernel(const float* __restrict__ x, const float* __restrict__ y
     const rsrc_t rgo = make_rsrc(go + e * NOC * C, NOC * row);
     const rsrc_t rdx = make_rsrc(dx ? dx + e * NX * C : nullptr, NX * row);
     const rsrc_t rdg = make_rsrc(dg ? dg + e * NP * C : nullptr, NP * row);
+    const rsrc_t rw = make_rsrc(w, NP * row);
     float dyl[NY];
 #pragma unroll
     for (int j = 0; j < NY; ++j) dyl[j] = 0.f;
@@ -358,13 +399,14 @@ tp_backward_wide_kernel(const float* __restrict__ x, const float* __restrict__ y
       const uint32_t vo = static_cast<uint32_t>(c) * 4u;
       const float* __restrict__ bond = opaque_lds_row(&sM[le][0]);
       constexpr int D = kBwdPrefetch;
-      float pre_g[D];                      // rows of the next D paths, in flight
+      float pre_g[D], pre_w[D];            // rows of the next D paths, in flight
       float pre_o[D][2 * LOUT + 1];
       auto request = [&](auto Q) {
         constexpr int q = Q;
         if constexpr (q < NP) {
           constexpr int nq = 2 * PS::tab.l3[q] + 1, oq = PS::tab.out[q];
           pre_g[q % D] = buf_load<1, kNonTemporal>(rg, vo + q * row).v[0];
+          if constexpr (WEIGHTED) pre_w[q % D] = buf_load<1>(rw, vo + q * row).v[0];
           static_for<0, nq>([&](auto K) { pre_o[q % D][K] = buf_load<1, kNonTemporal>(rgo, vo + (oq + K) * row).v[0]; });
         }
       };
@@ -390,7 +432,8 @@ tp_backward_wide_kernel(const float* __restrict__ x, const float* __restrict__ y
           constexpr int nj = 2 * l2 + 1, no = 2 * l3 + 1;
           constexpr int boff = PS::tab.bond[p];
           using CG = CGTab<a, l2, l3>;
-          const float gv = pre_g[p % D];
+          const float wv = WEIGHTED ? pre_w[p % D] : 1.f;
+          const float gv = WEIGHTED ? pre_g[p % D] * wv : pre_g[p % D];
           float o[no];
           static_for<0, no>([&](auto K) { o[K] = pre_o[p % D][K]; });
           request(Int<p + D>{});           // issued ahead of this path's dg store
@@ -406,7 +449,7 @@ tp_backward_wide_kernel(const float* __restrict__ x, const float* __restrict__ y
             });
             dgv = fmaf(base, o[K], dgv);
           });
-          buf_store<1>(rdg, vo + p * row, Vec<1>{{dgv}});
+          buf_store<1>(rdg, vo + p * row, Vec<1>{{WEIGHTED ? dgv * wv : dgv}});
           float part[nj];
 #pragma unroll
           for (int j = 0; j < nj; ++j) part[j] = 0.f;
@@ -432,41 +475,60 @@ tp_backward_wide_kernel(const float* __restrict__ x, const float* __restrict__ y
 }
 
 // ----------------------------------------------------------------------------- launchers
-using FwdLaunch = int (*)(const ictc_tp_desc&, const float*, const float*, const float*, float*,
+// w: the frozen path weight [P, C], or null.
+using FwdLaunch = int (*)(const ictc_tp_desc&, const float*, const float*, const float*, const float*, float*,
                           int64_t, hipStream_t);
-using BwdLaunch = int (*)(const ictc_tp_desc&, const float*, const float*, const float*,
+using BwdLaunch = int (*)(const ictc_tp_desc&, const float*, const float*, const float*, const float*,
                           const float*, float*, float*, float*, int64_t, hipStream_t);
 
 inline int launch_status() { return hipGetLastError() == hipSuccess ? ICTC_OK : ICTC_ERR_LAUNCH; }
 
-template <int LIN, int LE, int LOUT>
-int launch_forward(const ictc_tp_desc& d, const float* x, const float* y, const float* g, float* out,
-                   int64_t rows, hipStream_t stream) {
+template <int LIN, int LE, int LOUT, int NV, bool WEIGHTED>
+int launch_forward_as(const ictc_tp_desc& d, const float* x, const float* y, const float* g, const float* w, float* out,
+                      int64_t rows, hipStream_t stream) {
   const dim3 grid(static_cast<unsigned>((rows + kFwdTile - 1) / kFwdTile));
-  if (d.channels % (2 * kWave) == 0)
-    hipLaunchKernelGGL((tp_forward_kernel<LIN, LE, LOUT, 2>), grid, dim3(kBlock), 0, stream, x, y, g,
-                       out, d, rows);
-  else
-    hipLaunchKernelGGL((tp_forward_kernel<LIN, LE, LOUT, 1>), grid, dim3(kBlock), 0, stream, x, y, g,
-                       out, d, rows);
+  const size_t lds = WEIGHTED ? sizeof(float) * d.num_paths * d.channels : 0;
+  hipLaunchKernelGGL((tp_forward_kernel<LIN, LE, LOUT, NV, WEIGHTED>), grid, dim3(kBlock), lds, stream, x, y, g, w, out,
+                     d, rows);
   return launch_status();
 }
 
 template <int LIN, int LE, int LOUT>
-int launch_backward(const ictc_tp_desc& d, const float* x, const float* y, const float* g,
-                    const float* go, float* dx, float* dy, float* dg, int64_t rows, hipStream_t stream) {
-  const dim3 grid(static_cast<unsigned>((rows + kBwdTile - 1) / kBwdTile));
+int launch_forward(const ictc_tp_desc& d, const float* x, const float* y, const float* g, const float* w, float* out,
+                   int64_t rows, hipStream_t stream) {
+  if (d.channels % (2 * kWave) == 0)
+    return w ? launch_forward_as<LIN, LE, LOUT, 2, true>(d, x, y, g, w, out, rows, stream)
+             : launch_forward_as<LIN, LE, LOUT, 2, false>(d, x, y, g, w, out, rows, stream);
+  return w ? launch_forward_as<LIN, LE, LOUT, 1, true>(d, x, y, g, w, out, rows, stream)
+           : launch_forward_as<LIN, LE, LOUT, 1, false>(d, x, y, g, w, out, rows, stream);
+}
+
+template <int LIN, int LE, int LOUT, int NV, bool WEIGHTED>
+int launch_backward_as(const ictc_tp_desc& d, const float* x, const float* y, const float* g, const float* w,
+                       const float* go, float* dx, float* dy, float* dg, int64_t rows, hipStream_t stream) {
   if constexpr (LIN >= 4) {
     if (rows > 0x7fffffff) return ICTC_ERR_INVALID_ARGUMENT;   // one workgroup per instance
-    hipLaunchKernelGGL((tp_backward_wide_kernel<LIN, LE, LOUT>), dim3(static_cast<unsigned>(rows)),
-                       dim3(kWideBlock), 0, stream, x, y, g, go, dx, dy, dg, d, rows);
-  } else if (d.channels % (2 * kWave) == 0)
-    hipLaunchKernelGGL((tp_backward_kernel<LIN, LE, LOUT, 2>), grid, dim3(kBlock), 0, stream, x, y, g,
+    hipLaunchKernelGGL((tp_backward_wide_kernel<LIN, LE, LOUT, WEIGHTED>), dim3(static_cast<unsigned>(rows)),
+                       dim3(kWideBlock), 0, stream, x, y, g, w, go, dx, dy, dg, d, rows);
+  } else {
+    const dim3 grid(static_cast<unsigned>((rows + kBwdTile - 1) / kBwdTile));
+    const size_t lds = WEIGHTED ? sizeof(float) * d.num_paths * d.channels : 0;
+    hipLaunchKernelGGL((tp_backward_kernel<LIN, LE, LOUT, NV, WEIGHTED>), grid, dim3(kBlock), lds, stream, x, y, g, w,
                        go, dx, dy, dg, d, rows);
-  else
-    hipLaunchKernelGGL((tp_backward_kernel<LIN, LE, LOUT, 1>), grid, dim3(kBlock), 0, stream, x, y, g,
-                       go, dx, dy, dg, d, rows);
+  }
   return launch_status();
+}
+
+template <int LIN, int LE, int LOUT>
+int launch_backward(const ictc_tp_desc& d, const float* x, const float* y, const float* g, const float* w,
+                    const float* go, float* dx, float* dy, float* dg, int64_t rows, hipStream_t stream) {
+  if constexpr (LIN < 4) {
+    if (d.channels % (2 * kWave) == 0)
+      return w ? launch_backward_as<LIN, LE, LOUT, 2, true>(d, x, y, g, w, go, dx, dy, dg, rows, stream)
+               : launch_backward_as<LIN, LE, LOUT, 2, false>(d, x, y, g, w, go, dx, dy, dg, rows, stream);
+  }
+  return w ? launch_backward_as<LIN, LE, LOUT, 1, true>(d, x, y, g, w, go, dx, dy, dg, rows, stream)
+           : launch_backward_as<LIN, LE, LOUT, 1, false>(d, x, y, g, w, go, dx, dy, dg, rows, stream);
 }
 
 }  // namespace ictc

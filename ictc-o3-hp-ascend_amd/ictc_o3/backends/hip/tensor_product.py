@@ -82,6 +82,7 @@ class TensorProductPlan:
             desc.out_offset[s] = offsets[s]
             desc.scale[s] = self.plan.scales[index[p]] if p in index else 0.0
         self.desc = desc
+        self._weight_capacity = None
         self.num_paths = len(paths)
         self.full_paths = full
         self.is_full = paths == full
@@ -101,30 +102,37 @@ class TensorProductPlan:
                         rows.extend(range(offsets[s], offsets[s] + 2 * l + 1))
             self.output_rows = rows
 
+    @property
+    def weight_capacity(self) -> int:
+        """Widest path weight (floats) the degree set's kernels fold into the gates (0: none)."""
+        if self._weight_capacity is None:
+            self._weight_capacity = max(0, int(_lib.lib().ictc_hip_tp_weight_capacity(ctypes.byref(self.desc))))
+        return self._weight_capacity
+
     def set_scale(self, path_index: int, value: float) -> None:
         self.desc.scale[self.full_paths.index(self.paths[path_index])] = float(value)
 
 
-def _forward_raw(plan: TensorProductPlan, x, y, g) -> torch.Tensor:
+def _forward_raw(plan: TensorProductPlan, x, y, g, w=None) -> torch.Tensor:
+    """w: a frozen path weight [P*C] folded into the gates by the kernel (``weight_capacity``)."""
     rows = x.shape[0]
     out = torch.empty(rows, plan.full_out_width, device=x.device, dtype=torch.float32)
-    _lib.check(_lib.lib().ictc_hip_tp_forward(ctypes.byref(plan.desc), x.data_ptr(), y.data_ptr(),
-                                               g.data_ptr(), out.data_ptr(), rows,
-                                               _lib.stream_of(x.device)), "ictc_hip_tp_forward")
+    _lib.check(_lib.lib().ictc_hip_tp_forward_weighted(
+        ctypes.byref(plan.desc), x.data_ptr(), y.data_ptr(), g.data_ptr(), _lib.ptr(w), out.data_ptr(), rows,
+        _lib.stream_of(x.device)), "ictc_hip_tp_forward_weighted")
     return out
 
 
-def _backward_raw(plan: TensorProductPlan, need, x, y, g, go):
+def _backward_raw(plan: TensorProductPlan, need, x, y, g, go, w=None):
     rows = go.shape[0]
     dev = go.device
     dx = torch.empty(rows, plan.x_width, device=dev, dtype=torch.float32) if need[0] else None
     dy = torch.empty(rows, plan.y_width, device=dev, dtype=torch.float32) if need[1] else None
     dg = torch.empty(rows, plan.full_gate_width, device=dev, dtype=torch.float32) if need[2] else None
     if any(need):
-        _lib.check(_lib.lib().ictc_hip_tp_backward(
-            ctypes.byref(plan.desc), x.data_ptr(), y.data_ptr(),
-            g.data_ptr(), go.data_ptr(), _lib.ptr(dx), _lib.ptr(dy), _lib.ptr(dg), rows,
-            _lib.stream_of(dev)), "ictc_hip_tp_backward")
+        _lib.check(_lib.lib().ictc_hip_tp_backward_weighted(
+            ctypes.byref(plan.desc), x.data_ptr(), y.data_ptr(), g.data_ptr(), _lib.ptr(w), go.data_ptr(),
+            _lib.ptr(dx), _lib.ptr(dy), _lib.ptr(dg), rows, _lib.stream_of(dev)), "ictc_hip_tp_backward_weighted")
     return dx, dy, dg
 
 
@@ -135,31 +143,34 @@ def _add(acc, value):
 
 
 class _Forward(torch.autograd.Function):
+    """w: a frozen path weight folded into the gates, or None (a constant of the map: the map and
+    every derivative of it stay trilinear in x, Y and g)."""
+
     @staticmethod
-    def forward(ctx, plan, x, y, g):
+    def forward(ctx, plan, x, y, g, w=None):
         ctx.plan = plan
-        ctx.save_for_backward(x, y, g)
-        return _forward_raw(plan, x, y, g)
+        ctx.save_for_backward(x, y, g, w)
+        return _forward_raw(plan, x, y, g, w)
 
     @staticmethod
     def backward(ctx, go):
-        x, y, g = ctx.saved_tensors
-        need = required_gradients((x, y, g), ctx.needs_input_grad[1:])
+        x, y, g, w = ctx.saved_tensors
+        need = required_gradients((x, y, g), ctx.needs_input_grad[1:4])
         if go is None or not any(need):
-            return None, None, None, None
-        dx, dy, dg = vjp(ctx.plan, need, x, y, g, go.contiguous())
-        return None, dx, dy, dg
+            return None, None, None, None, None
+        dx, dy, dg = vjp(ctx.plan, need, x, y, g, go.contiguous(), w)
+        return None, dx, dy, dg, None
 
 
 class _Backward(torch.autograd.Function):
     """(dx, dY, dg) = VJP(x, Y, g; go); outputs not requested are empty placeholders."""
 
     @staticmethod
-    def forward(ctx, plan, need, x, y, g, go):
+    def forward(ctx, plan, need, x, y, g, go, w=None):
         ctx.plan, ctx.need = plan, need
         ctx.set_materialize_grads(False)
-        ctx.save_for_backward(x, y, g, go)
-        dx, dy, dg = _backward_raw(plan, need, x, y, g, go)
+        ctx.save_for_backward(x, y, g, go, w)
+        dx, dy, dg = _backward_raw(plan, need, x, y, g, go, w)
         empty = go.new_empty(0)
         outs = tuple(t if t is not None else empty for t in (dx, dy, dg))
         for t, n in zip(outs, need):
@@ -170,53 +181,54 @@ class _Backward(torch.autograd.Function):
     @staticmethod
     def backward(ctx, hx, hy, hg):
         plan, need_out = ctx.plan, ctx.need
-        x, y, g, go = ctx.saved_tensors
+        x, y, g, go, w = ctx.saved_tensors
         hx = hx if need_out[0] else None
         hy = hy if need_out[1] else None
         hg = hg if need_out[2] else None
-        nx, ny, ng, no = required_gradients((x, y, g, go), ctx.needs_input_grad[2:])
+        nx, ny, ng, no = required_gradients((x, y, g, go), ctx.needs_input_grad[2:6])
         gx = gy = gg = ggo = None
         if hx is not None:
             hx = hx.contiguous()
             if ny or ng:
-                _, a, b = vjp(plan, (False, ny, ng), hx, y, g, go)
+                _, a, b = vjp(plan, (False, ny, ng), hx, y, g, go, w)
                 gy, gg = _add(gy, a), _add(gg, b)
             if no:
-                ggo = _add(ggo, _Forward.apply(plan, hx, y, g))
+                ggo = _add(ggo, _Forward.apply(plan, hx, y, g, w))
         if hy is not None:
             hy = hy.contiguous()
             if nx or ng:
-                a, _, b = vjp(plan, (nx, False, ng), x, hy, g, go)
+                a, _, b = vjp(plan, (nx, False, ng), x, hy, g, go, w)
                 gx, gg = _add(gx, a), _add(gg, b)
             if no:
-                ggo = _add(ggo, _Forward.apply(plan, x, hy, g))
+                ggo = _add(ggo, _Forward.apply(plan, x, hy, g, w))
         if hg is not None:
             hg = hg.contiguous()
             if nx or ny:
-                a, b, _ = vjp(plan, (nx, ny, False), x, y, hg, go)
+                a, b, _ = vjp(plan, (nx, ny, False), x, y, hg, go, w)
                 gx, gy = _add(gx, a), _add(gy, b)
             if no:
-                ggo = _add(ggo, _Forward.apply(plan, x, y, hg))
-        return None, None, gx, gy, gg, ggo
+                ggo = _add(ggo, _Forward.apply(plan, x, y, hg, w))
+        return None, None, gx, gy, gg, ggo, None
 
 
-def vjp(plan, need, x, y, g, go):
+def vjp(plan, need, x, y, g, go, w=None):
     """(dx, dY, dg) with None for entries not in ``need``; differentiable."""
     need = tuple(bool(n) for n in need)
     if not any(need):
         return None, None, None
     if not torch.is_grad_enabled():       # nothing recorded: skip the autograd Function
-        return _backward_raw(plan, need, x, y, g, go)
-    outs = _Backward.apply(plan, need, x, y, g, go)
+        return _backward_raw(plan, need, x, y, g, go, w)
+    outs = _Backward.apply(plan, need, x, y, g, go, w)
     return tuple(o if n else None for o, n in zip(outs, need))
 
 
 def packed_tensor_product(plan: TensorProductPlan, features: torch.Tensor, harmonics: torch.Tensor,
-                          gates: torch.Tensor) -> torch.Tensor:
+                          gates: torch.Tensor, weight: Optional[torch.Tensor] = None) -> torch.Tensor:
     """Packed ir_mul TP: features [E, C(L_in+1)^2], harmonics [E,(L_e+1)^2],
-    gates [E, P*C] (path weights already folded in) -> [E, NOC*C]."""
+    gates [E, P*C] -> [E, NOC*C].  The path weights are folded into the gates already, or passed as
+    ``weight`` [P*C] for the kernels to fold (see ``gates_and_weight``)."""
     if plan.is_full:
-        return _Forward.apply(plan, features.contiguous(), harmonics.contiguous(), gates.contiguous())
+        return _Forward.apply(plan, features.contiguous(), harmonics.contiguous(), gates.contiguous(), weight)
     rows, c = gates.shape[0], plan.channels
     slots = torch.tensor(plan.slot_of_path, device=gates.device)
     full_gates = gates.new_zeros(rows, len(plan.full_paths), c).index_copy(
@@ -225,6 +237,19 @@ def packed_tensor_product(plan: TensorProductPlan, features: torch.Tensor, harmo
                          full_gates.reshape(rows, len(plan.full_paths) * c))
     keep = torch.tensor(plan.output_rows, device=gates.device)
     return out.reshape(rows, -1, c).index_select(1, keep).reshape(rows, len(plan.output_rows) * c)
+
+
+def gates_and_weight(owner, plan: TensorProductPlan, gates: Optional[torch.Tensor], rows: int):
+    """(gates [E, P*C], path weight [P*C] or None) for ``packed_tensor_product``: the owner's
+    per-(path, channel) weight is left to the kernels when nothing differentiates it and they take it
+    (every path of a compiled degree set, P*C up to ``weight_capacity``), which saves a pass over the
+    gates and one over their gradients; otherwise it is multiplied into the gates here
+    (``owner.effective_gates``).  Both read the weight on every call and round the same products."""
+    w = owner.weight
+    if (gates is None or not plan.is_full or plan.full_gate_width > plan.weight_capacity
+            or w.device != gates.device or (w.requires_grad and torch.is_grad_enabled())):
+        return owner.effective_gates(gates, rows), None
+    return gates.reshape(rows, plan.full_gate_width), w.detach().reshape(-1).contiguous()
 
 
 def blocks_to_packed(blocks: Dict[int, torch.Tensor], lmax: int) -> torch.Tensor:
@@ -292,7 +317,8 @@ def tensor_product(owner, features, harmonics, gates=None):
     x = pack_features(owner, features, rows)
     y = pack_harmonics(owner, harmonics, rows, sample)
     plan = owner.hip_plan(*owner_degrees(owner))
-    return packed_to_blocks(plan, packed_tensor_product(plan, x, y, owner.effective_gates(gates, rows)))
+    gates, weight = gates_and_weight(owner, plan, gates, rows)
+    return packed_to_blocks(plan, packed_tensor_product(plan, x, y, gates, weight))
 
 
 def destination_nodes(owner, source_nodes: int) -> int:

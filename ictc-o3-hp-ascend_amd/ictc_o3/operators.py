@@ -148,14 +148,14 @@ class EdgeTensorProduct(torch.nn.Module):
         return rows
 
     def forward(self, features, harmonics, gates):
-        from ictc_o3.backends.hip.tensor_product import packed_tensor_product
+        from ictc_o3.backends.hip.tensor_product import gates_and_weight, packed_tensor_product
         rows = self._check(features, harmonics, gates)
         if not rows:
             zero = sum(v.sum() * 0 for v in (features, harmonics, self.tp.weight,
                                              *(() if gates is None else (gates,))))
             return features.new_empty(0, self.output_width) + zero
-        out = packed_tensor_product(self.plan, self._to_ir_mul_features(features), harmonics,
-                                    self.tp.effective_gates(gates, rows))
+        gates, weight = gates_and_weight(self.tp, self.plan, gates, rows)
+        out = packed_tensor_product(self.plan, self._to_ir_mul_features(features), harmonics, gates, weight)
         return self._from_ir_mul_output(out)
 
 

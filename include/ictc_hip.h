@@ -121,6 +121,22 @@ int ictc_hip_tp_backward(const ictc_tp_desc* desc,
                          int64_t rows, hipStream_t stream);
 
 /*
+ * The same two maps with a frozen per-(path, channel) weight [P, C] (null: none) folded into the gates
+ * by the kernels: out = TP(x, Y, g * w), grad_gates = w * d/d(g * w).  Bit-identical to a separate
+ * g * w pass (reference ictc_o3/backends/ascend/packed_tensor_product.py:163-164).  P * C at most
+ * ictc_hip_tp_weight_capacity(desc) (0: the degree set does not take a weight, -1: bad descriptor), else
+ * ICTC_ERR_UNSUPPORTED.
+ */
+int ictc_hip_tp_weight_capacity(const ictc_tp_desc *desc);
+int ictc_hip_tp_forward_weighted(const ictc_tp_desc *desc, const float *features, const float *harmonics,
+                                 const float *gates, const float *path_weight, float *out, int64_t rows,
+                                 hipStream_t stream);
+int ictc_hip_tp_backward_weighted(const ictc_tp_desc *desc, const float *features, const float *harmonics,
+                                  const float *gates, const float *path_weight, const float *grad_out,
+                                  float *grad_features, float *grad_harmonics, float *grad_gates, int64_t rows,
+                                  hipStream_t stream);
+
+/*
  * Graph message:  node_out[n] = sum_{e : dst(e) = n} TP(features[src(e)], harmonics[e], gates[e])
  * with the TP above (same descriptor; node rows use the features / output layouts).
  *

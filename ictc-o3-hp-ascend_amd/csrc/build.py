@@ -159,8 +159,10 @@ def _generate(combos) -> list:
         _write_if_changed(path, f'#include "sc_kernels.hpp"\n#include "generated/sc_{l}{t}{k}.hpp"\n'
                                 f'namespace ictc {{\ntemplate int launch_sc<{l}, {t}, {k}>(int, const float*, '
                                 'const float*, const int64_t*, const float*, const float*, float*, int, '
-                                'int64_t, int, '
-                                'hipStream_t);\n}  // namespace ictc\n')
+                                'int64_t, int, hipStream_t);\n'
+                                f'template int launch_sc_weight_grad<{l}, {t}, {k}>(const float*, const float*, '
+                                'const int64_t*, const int32_t*, const float*, float*, int, int64_t, int, int64_t, '
+                                'int, hipStream_t);\n}  // namespace ictc\n')
         units.append((os.path.getsize(os.path.join(GEN, f"sc_{l}{t}{k}.hpp")) // 20, path))
     units.sort(reverse=True)
     return [p for _, p in units]

@@ -420,7 +420,7 @@ def emit(lmax: int, target: int, corr: int) -> str:
         assert k == len(steps)
         return out
 
-    def loop(steps, decl, with_u=False):
+    def loop(steps, decl, with_u=False, stride='asm volatile("" : "+s"(Cs));'):
         # C, the input copy and (when used) the cotangent copy are re-laundered every
         # iteration, so that weight addresses and products of x or u with constants are
         # formed inside their step instead of being hoisted (all at once) out of the loop
@@ -429,7 +429,7 @@ def emit(lmax: int, target: int, corr: int) -> str:
             out.append(f"float ul[{NO}];\n  for (int i = 0; i < {NO}; ++i) ul[i] = u[i];")
         out += ["  #pragma clang loop unroll(disable)",
                 f"  for (int step = 0; step < {len(steps)}; ++step) {{",
-                '    int Cs = C;', '    asm volatile("" : "+s"(Cs));',
+                '    int Cs = C;', f'    {stride}',
                 f"    #pragma unroll\n    for (int i = 0; i < {D}; ++i) launder(xl[i]);"]
         if with_u:
             out.append(f"    #pragma unroll\n    for (int i = 0; i < {NO}; ++i) launder(ul[i]);")
@@ -448,7 +448,8 @@ def emit(lmax: int, target: int, corr: int) -> str:
         fw += ["  if constexpr (__is_same(V, float)) {"] + straight(fsteps, copy + zq + f"V P[{maxq}];")
         fw += ["  } else {"] + loop(merged(fsteps, fgroups), copy + zq + f"V P[{maxq}];") + ["  }"]
         bw += loop(merged(bsteps, bgroups), copy + zq + f"V P[{maxq}], G[{maxq}];", with_u=True)
-        aw += loop(merged(asteps, agroups), copy + f"V Q[{qn}];\n  V P[{maxq}];", with_u=True)
+        aw += loop(merged(asteps, agroups), copy + f"V Q[{qn}];\n  V P[{maxq}];", with_u=True,
+                   stride="launder(Cs, phi);")
     off_lines = ", ".join(str(offsets[(lo, o)]) for lo in range(target + 1) for o in range(corr, 0, -1))
     return "\n".join([
         f"// Generated by csrc/gen_sc.py for lmax={lmax}, target_lmax={target}, correlation={corr}.",
@@ -476,8 +477,9 @@ def emit(lmax: int, target: int, corr: int) -> str:
         "  // phi[p*C] = part(sum_m u_m chain_p(x)_m) for every weight column p (weight adjoint;",
         "  // part() is the value for float and the tangent for Dual)",
         "  template <typename V>",
+        "  // phi: the node's [KTOT, C] row, or sums in LDS that the assignments add to (LdsSums)",
         "  __device__ static __forceinline__ void weight_features(const V* x, int C, const float* u,",
-        "                                                         float* __restrict__ phi) {",
+        "                                                         auto phi) {",
         *aw,
         "  }",
         "};",

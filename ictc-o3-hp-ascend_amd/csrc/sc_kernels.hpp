@@ -126,6 +126,101 @@ sc_kernel(const float* __restrict__ x, const float* __restrict__ t, const int64_
   }
 }
 
+// Weight gradients dW[s, p, c] = sum over the nodes of species s of <u, chain_p(x)> (DUAL: of its
+// derivative along t), without the per-node features [N, KTOT, C] in memory: one wave per (range of
+// the nodes ordered by species, 64-channel chunk) adds each node's features into its LDS columns
+// [KTOT][64] and writes them out at the end of each species.  The species s of range r goes to
+// partial slot r + s: along the ordered nodes each next (range, species) pair raises one of the two, so
+// the slots are distinct.  sc_weight_sum_kernel adds a species' slots in order.
+// At C = 128, lmax 3 -> 0e+1o, 16,411 nodes: 131 us, and 15 + 10 us for the node order and the slot sums,
+// against 156 us for writing the features (0.72 GB) and 224 us for multiplying them with the species'
+// one-hot rows; bound by the VALU at under two waves per SIMD (the LDS columns' room).  KTOT up to kScWgColumns (24 KB of LDS: six waves
+// per CU); wider plans would leave the CUs with one or two waves and keep the features.
+constexpr int kScWgColumns = 96;
+
+// Node ranges per chunk: as many waves as fit the chip (by their LDS), four nodes each at least.
+inline int64_t sc_wg_ranges(int ktot, int C, int64_t nodes) {
+  const int64_t nchunks = (C + kWave - 1) / kWave;
+  int64_t per_cu = (160 * 1024) / (static_cast<int64_t>(ktot) * kWave * 4);
+  per_cu = per_cu < 16 ? per_cu : 16;
+  const int64_t want = (per_cu * compute_units() + nchunks - 1) / nchunks, most = (nodes + 3) / 4;
+  const int64_t r = want < most ? want : most;
+  return r < 1 ? 1 : r;
+}
+
+template <int L, int T, int K, bool DUAL>
+__global__ void __launch_bounds__(kWave)
+sc_weight_grad_kernel(const float* __restrict__ x, const float* __restrict__ t, const int64_t* __restrict__ species,
+                      const int32_t* __restrict__ order, const float* __restrict__ u, float* __restrict__ ws, int C,
+                      int64_t nodes, int num_species, int nchunks, int per_range) {
+  using PL = sc::Plan<L, T, K>;
+  constexpr int D = PL::D, NO = PL::NO, KT = PL::KTOT;
+  __shared__ float sums[KT * kWave];
+  const int lane = threadIdx.x;
+  const int range = blockIdx.x / nchunks, chunk = blockIdx.x - range * nchunks;
+  const int64_t i0 = static_cast<int64_t>(range) * per_range;
+  const int64_t i1 = i0 + per_range < nodes ? i0 + per_range : nodes;
+  const int c = chunk * kWave + lane;
+  const bool live = c < C;
+  const int cc = live ? c : 0;
+  struct In {
+    float x[D], t[DUAL ? D : 1], u[NO];
+    int s;
+  };
+  auto fetch = [&](int64_t i, In& in) {
+    const int64_t node = __builtin_amdgcn_readfirstlane(order[i]);
+    const int64_t s = species[node];
+    in.s = static_cast<int>(s < 0 || s >= num_species ? 0 : s);   // host validates, as sc_kernel
+    sc_load_mul_ir<L>(x + node * D * C, C, cc, live, in.x);
+    if constexpr (DUAL) sc_load_mul_ir<L>(t + node * D * C, C, cc, live, in.t);
+    sc_load_mul_ir<T>(u + node * NO * C, C, cc, live, in.u);
+  };
+  In cur;
+  fetch(i0, cur);
+  for (int p = 0; p < KT; ++p) sums[p * kWave + lane] = 0.f;
+  for (int64_t i = i0; i < i1; ++i) {
+    In next;
+    const bool more = i + 1 < i1;
+    if (more) fetch(i + 1, next);
+    const sc::LdsSums phi{sums + lane};
+    if constexpr (DUAL) {
+      sc::Dual xd[D];
+#pragma unroll
+      for (int m = 0; m < D; ++m) xd[m] = sc::Dual(cur.x[m], cur.t[m]);
+      PL::weight_features(xd, kWave, cur.u, phi);
+    } else {
+      PL::weight_features(cur.x, kWave, cur.u, phi);
+    }
+    if (!more || next.s != cur.s) {   // wave-uniform: the species' last node of this range
+      float* __restrict__ out = ws + static_cast<int64_t>(range + cur.s) * KT * C + cc;
+      for (int p = 0; p < KT; ++p) {
+        if (live) out[static_cast<int64_t>(p) * C] = sums[p * kWave + lane];
+        sums[p * kWave + lane] = 0.f;
+      }
+    }
+    if (more) cur = next;
+  }
+}
+
+template <int L, int T, int K>
+int launch_sc_weight_grad(const float* x, const float* t, const int64_t* species, const int32_t* order, const float* u,
+                          float* ws, int C, int64_t nodes, int num_species, int64_t ranges, int per_range,
+                          hipStream_t stream) {
+  if constexpr (sc::Plan<L, T, K>::KTOT > kScWgColumns) {
+    return ICTC_ERR_UNSUPPORTED;
+  } else {
+    const int nchunks = (C + kWave - 1) / kWave;
+    const dim3 grid(static_cast<unsigned>(ranges * nchunks));
+    if (t != nullptr)
+      hipLaunchKernelGGL((sc_weight_grad_kernel<L, T, K, true>), grid, dim3(kWave), 0, stream, x, t, species, order, u,
+                         ws, C, nodes, num_species, nchunks, per_range);
+    else
+      hipLaunchKernelGGL((sc_weight_grad_kernel<L, T, K, false>), grid, dim3(kWave), 0, stream, x, t, species, order, u,
+                         ws, C, nodes, num_species, nchunks, per_range);
+    return hipGetLastError() == hipSuccess ? ICTC_OK : ICTC_ERR_LAUNCH;
+  }
+}
+
 template <int L, int T, int K>
 int launch_sc(int mode, const float* x, const float* t, const int64_t* species, const float* w,
               const float* u, float* out, int C, int64_t nodes, int num_species, hipStream_t stream) {

@@ -44,6 +44,22 @@ __device__ __forceinline__ void launder(Dual& a) {
   asm volatile("" : "+v"(a.d));
 }
 
+// Sums of the weight features over several nodes, one LDS column per lane ([KTOT][64] floats of the wave):
+// the generated assignment phi[p * Cs] = v adds v to the lane's sum of column p.  Cs stays the
+// compile-time stride, so that every column has an immediate LDS offset.
+struct LdsSums {
+  float* p;
+  struct Ref {
+    float* at;
+    __device__ __forceinline__ void operator=(float v) const { *at += v; }
+  };
+  __device__ __forceinline__ Ref operator[](int i) const { return {p + i}; }
+};
+
+// the stride of a node's phi row, opaque like the inputs (row addresses formed inside their step)
+__device__ __forceinline__ void launder(int& stride, float*) { asm volatile("" : "+s"(stride)); }
+__device__ __forceinline__ void launder(int&, LdsSums) {}
+
 template <int L, int T, int K>
 struct Plan;
 

@@ -7,15 +7,17 @@ prefixes (see ictc_o3/basis/symmetric_u.py).  Gradients:
 
 * node features: the ``ictc_hip_sc_backward`` kernel;
 * weights: the map is linear in W, so dW[s] is the sum over the nodes of species s
-  of the per-node chain features <u, chain_p(x)> (``ictc_hip_sc_weight_features``),
-  reduced by species as one GEMM with the species one-hot matrix.
+  of the per-node chain features <u, chain_p(x)>: summed in one pass
+  (``ictc_hip_sc_weight_grad``), or for plans of more than 96 weight columns written out
+  (``ictc_hip_sc_weight_features``) and reduced by one GEMM with the species one-hot matrix.
 
 The backward is itself a differentiable Function (second derivatives, as force
 training needs).  With cotangents (a, B) of (dx, dW):
   d/d go = J(x) a + forward(x, B)
   d/d x  = H_go(x) a + vjp(x, B, go)
   d/d W  = species-sum of <go, d chain_p(x)[a]>
-through the directional kernels (``ictc_hip_sc_jvp``, ``_hvp``, ``_weight_features_jvp``);
+through the directional kernels (``ictc_hip_sc_jvp``, ``_hvp``, ``_weight_features_jvp``, and
+``_weight_grad`` with a tangent);
 third derivatives are not provided.
 """
 from __future__ import annotations
@@ -68,8 +70,28 @@ def _species_sum(plan: ContractionPlan, species, phi):
         plan.num_elements, plan.ktot, plan.channels)
 
 
+def _weight_grad_fused(plan: ContractionPlan, x, species, go, t=None):
+    """dW [S, KTOT, C] in one pass over the nodes (t: its derivative along the tangent t), or None for
+    a plan the kernel does not cover (``ictc_hip_sc_weight_grad``: up to 96 weight columns)."""
+    lib, n = _lib.lib(), x.shape[0]
+    floats = int(lib.ictc_hip_sc_weight_grad_workspace(plan.lmax, plan.target_lmax, plan.correlation, plan.channels,
+                                                       plan.num_elements, n))
+    if floats <= 0:
+        return None
+    ws = torch.empty(floats, device=x.device, dtype=torch.float32)
+    out = torch.empty(plan.num_elements, plan.ktot, plan.channels, device=x.device, dtype=torch.float32)
+    _lib.check(lib.ictc_hip_sc_weight_grad(
+        plan.lmax, plan.target_lmax, plan.correlation, plan.channels, x.data_ptr(), species.data_ptr(),
+        plan.num_elements, go.data_ptr(), _lib.ptr(t), ws.data_ptr(), floats, out.data_ptr(), n,
+        _lib.stream_of(x.device)), "ictc_hip_sc_weight_grad")
+    return out
+
+
 def _weight_grad(plan: ContractionPlan, x, species, go):
     """dW[s,p,c] = sum_{n: s_n = s} <go[n,c], chain_p(x[n,c])>."""
+    fused = _weight_grad_fused(plan, x, species, go)
+    if fused is not None:
+        return fused
     phi = torch.empty(x.shape[0], plan.ktot, plan.channels, device=x.device, dtype=torch.float32)
     _lib.check(_lib.lib().ictc_hip_sc_weight_features(
         plan.lmax, plan.target_lmax, plan.correlation, plan.channels, x.data_ptr(), species.data_ptr(),
@@ -98,6 +120,9 @@ def _hvp_raw(plan: ContractionPlan, x, species, w, go, t):
 
 def _weight_grad_jvp(plan: ContractionPlan, x, species, go, t):
     """sum over the nodes of each species of <go[n,c], d chain_p(x[n,c])[t[n,c]]>."""
+    fused = _weight_grad_fused(plan, x, species, go, t)
+    if fused is not None:
+        return fused
     phi = torch.empty(x.shape[0], plan.ktot, plan.channels, device=x.device, dtype=torch.float32)
     _lib.check(_lib.lib().ictc_hip_sc_weight_features_jvp(
         plan.lmax, plan.target_lmax, plan.correlation, plan.channels, x.data_ptr(), species.data_ptr(),

@@ -350,6 +350,20 @@ int ictc_hip_sc_weight_features_jvp(int lmax, int target_lmax, int correlation, 
                                     float* features_out, int64_t nodes, hipStream_t stream);
 
 /*
+ * Weight gradients in one pass, without the per-node features: grad_weights[s, p, c] = sum over the nodes of
+ * species s of <grad_out, chain_p(x)> (tangent null) or of its derivative along the tangent (as
+ * _weight_features_jvp), summed in a fixed order; every entry is written, zero for a species without nodes.
+ * workspace: _workspace() floats (0: the plan is not covered, use _weight_features; negative:
+ * -ictc_status).
+ */
+int64_t ictc_hip_sc_weight_grad_workspace(int lmax, int target_lmax, int correlation, int channels, int num_elements,
+                                          int64_t nodes);
+int ictc_hip_sc_weight_grad(int lmax, int target_lmax, int correlation, int channels, const float *node_features,
+                            const int64_t *species, int num_elements, const float *grad_out, const float *tangent,
+                            float *workspace, int64_t workspace_floats, float *grad_weights, int64_t nodes,
+                            hipStream_t stream);
+
+/*
  * Direction harmonics (ICTC basis, component-normalised) and their analytic
  * derivative contractions, one thread per direction.
  *   directions [rows, 3]; Y has (lmax+1)^2 components Y_0 | Y_1 | ...

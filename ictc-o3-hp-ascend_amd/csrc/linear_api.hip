@@ -1,4 +1,4 @@
-// Per-degree channel linear on fp32 MFMA (gfx950): the path-preserving message linear of the
+// Per-degree channel linear on the matrix cores (gfx950): the path-preserving message linear of the
 // MACE interaction (reference mace_ictc/models/pure_cartesian_ictd_fix.py:629-661,
 // PathPreservingLinearSO3; native route ictc_o3/ascendc/linear.py:12-136), applied straight to
 // the message kernel's packed output and writing the mul_ir node layout.
@@ -14,6 +14,9 @@
 // the layout changes folded into the tile loads and stores (no transposed copies, no
 // concatenation, the 1/avg_num_neighbors scale as alpha).
 //
+// Calls that give every CU a block run on the bf16 matrix cores with fp32 operands in three parts (the split
+// kernels below), the weight gradient always; smaller calls on fp32 MFMA, in more and smaller blocks:
+//
 // Tiling: a 256-thread block computes a 64-row x 64-column output tile of one degree (grid.z);
 // K is walked in chunks of 32 staged through LDS, then each wave runs v_mfma_f32_16x16x4_f32 over
 // its 16 rows and the tile's 4 column tiles.  Operand layout of that instruction: lane l supplies
@@ -27,6 +30,7 @@
 
 #include "ictc_common.hpp"
 #include "ictc_hip.h"
+#include "split_bf16.hpp"
 
 namespace ictc {
 namespace {
@@ -283,6 +287,282 @@ degree_linear_kernel(const float* __restrict__ in, float* __restrict__ out, cons
   }
 }
 
+// The maps that write y on the bf16 matrix cores, fp32 operands in three parts (split_bf16.hpp): 64 rows x TN
+// columns per block (one 64 x 128 block reads each row once where the fp32 kernel's 64-column tiles read
+// it twice), K in chunks of 32.  Both operands are split when a chunk is staged: a thread holds
+// eight consecutive k of a row or column, one 16-byte LDS unit per part, in the operand order
+// [part][octet of k][row or column]; the next chunk's loads are in flight during the current one's
+// matrix instructions (two LDS buffers, one barrier per chunk).  Wave w computes rows 32 (w % 2) ..
+// and columns (TN / 2) (w / 2) ..  The small part products have accumulators of their own.
+// Bound by the staging between barriers at two blocks per CU.  2048 nodes, C = O = 128, counts (4, 6, 7, 6)
+// (19.9 GFLOP over forward and both adjoints): 51 us, on fp32 MFMA 75 us; error against float64 1.6e-7, 5.0e-7
+// there.  One LDS buffer with two barriers per chunk (three blocks per CU): 61 us.
+constexpr int kSpRows = kTile + 2;       // units per octet row: staggers the staging writes' banks
+
+template <int N>
+struct SplitTile {
+  bf16x8 v[3][kKc / 8][N];
+};
+
+template <int MODE, int TN>
+__global__ void __launch_bounds__(256, 2)
+degree_linear_split_kernel(const float* __restrict__ in, float* __restrict__ out, const LinearArgs a) {
+  static_assert(MODE != kInputGrad, "degree_linear_input_grad_kernel");
+  constexpr bool BT = MODE == kMulIrT;
+  constexpr bool STRIDED = MODE != kForward;
+  constexpr int NCT = TN / 64;           // 32-column tiles per wave
+  constexpr int NBT = TN / 64;           // octets of B per thread
+  const DegreeGeometry g = a.g[blockIdx.z];
+  const int d = g.d;
+  const int ncols = a.out_channels, kdim = g.k;
+  const int64_t r0 = static_cast<int64_t>(blockIdx.x) * kTile;
+  const int c0 = blockIdx.y * TN;
+  if (r0 >= g.rows || c0 >= ncols) return;
+  __shared__ SplitTile<kSpRows> sA[2];
+  __shared__ SplitTile<TN + 2> sB[2];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int C = a.channels;
+  const int ar = tid >> 2, ao = tid & 3, akq = ao * 8;   // A: row ar, octet ao
+  const int64_t arho = r0 + ar;
+  const int64_t an = arho < g.rows ? arho / d : 0;   // rows past the end read row 0; not stored
+  const int am = arho < g.rows ? static_cast<int>(arho - an * d) : 0;
+  const float* __restrict__ abase = in + an * a.xwidth + g.xoff + (STRIDED ? am : static_cast<int64_t>(am) * C);
+  float ra[8], rb[NBT][8];
+  auto fetch = [&](int k0) {
+    if constexpr (STRIDED) {
+      const float* p = abase + (k0 + akq) * d;
+#pragma unroll
+      for (int u = 0; u < 8; ++u) ra[u] = p[u * d];
+    } else {
+      const int blk = k0 / C, c = k0 - blk * C + akq;
+      const float* p = abase + blk * d * C + c;
+      const f32x4_t lo = *reinterpret_cast<const f32x4_t*>(p), hi = *reinterpret_cast<const f32x4_t*>(p + 4);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) ra[u] = lo[u], ra[4 + u] = hi[u];
+    }
+#pragma unroll
+    for (int q = 0; q < NBT; ++q) {
+      if constexpr (!BT) {   // weight row of column 64 q + tid / 4, its octet tid % 4
+        const int col = c0 + 64 * q + ar < ncols ? c0 + 64 * q + ar : ncols - 1;   // (not stored)
+        const float* p = g.w + static_cast<int64_t>(col) * g.k + k0 + akq;
+        const f32x4_t lo = *reinterpret_cast<const f32x4_t*>(p), hi = *reinterpret_cast<const f32x4_t*>(p + 4);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) rb[q][u] = lo[u], rb[q][4 + u] = hi[u];
+      } else {               // column 64 q + tid % 64, octet tid / 64: eight weight rows
+        const int col = c0 + 64 * q + (tid & 63) < ncols ? c0 + 64 * q + (tid & 63) : ncols - 1;
+        const float* p = g.w + static_cast<int64_t>(k0 + 8 * (tid >> 6)) * ncols + col;
+#pragma unroll
+        for (int u = 0; u < 8; ++u) rb[q][u] = p[static_cast<int64_t>(u) * ncols];
+      }
+    }
+  };
+  auto stage = [&](int buf) {
+    const Split8 sa = split8(ra);
+#pragma unroll
+    for (int q = 0; q < 3; ++q) sA[buf].v[q][ao][ar] = sa.p[q];
+#pragma unroll
+    for (int t = 0; t < NBT; ++t) {
+      const Split8 sb = split8(rb[t]);
+#pragma unroll
+      for (int q = 0; q < 3; ++q) {
+        if constexpr (!BT)
+          sB[buf].v[q][ao][64 * t + ar] = sb.p[q];
+        else
+          sB[buf].v[q][tid >> 6][64 * t + (tid & 63)] = sb.p[q];
+      }
+    }
+  };
+  const int r = lane & 31, half = lane >> 5, row_t = (wave & 1) * 32, col_t = (wave >> 1) * (TN / 2);
+  f32x16 hi[1][NCT], lo[1][NCT];
+#pragma unroll
+  for (int t = 0; t < NCT; ++t)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) hi[0][t][i] = lo[0][t][i] = 0.f;
+  if (kdim > 0) {   // uniform; a degree without path blocks writes its zero forward rows
+    fetch(0);
+    stage(0);
+    __syncthreads();
+    int buf = 0;
+    for (int k0 = 0; k0 < kdim; k0 += kKc) {
+      const bool more = k0 + kKc < kdim;
+      if (more) fetch(k0 + kKc);
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        Split8 av[1], bv[NCT];
+#pragma unroll
+        for (int q = 0; q < 3; ++q) av[0].p[q] = sA[buf].v[q][2 * k + half][row_t + r];
+#pragma unroll
+        for (int t = 0; t < NCT; ++t)
+#pragma unroll
+          for (int q = 0; q < 3; ++q) bv[t].p[q] = sB[buf].v[q][2 * k + half][col_t + 32 * t + r];
+        mfma_split(av, bv, hi, lo);
+      }
+      if (more) stage(buf ^ 1);
+      __syncthreads();
+      buf ^= 1;
+    }
+  }
+#pragma unroll
+  for (int t = 0; t < NCT; ++t) {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) hi[0][t][i] += lo[0][t][i];
+    const int col = c0 + col_t + 32 * t + r;
+    const bool redo = any_nonfinite(hi[0][t]);   // see split_bf16.hpp: these results again in fp32
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {   // four consecutive rows: one division, then (n, m) stepped
+      const int64_t rho0 = r0 + row_t + mfma_row(4 * q, half);
+      int64_t n = rho0 / d;
+      int m = static_cast<int>(rho0 - n * d);
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        if (v > 0 && ++m == d) {
+          m = 0;
+          ++n;
+        }
+        if (rho0 + v >= g.rows || col >= ncols) continue;
+        float val = hi[0][t][4 * q + v];
+        if (redo) {
+          val = 0.f;
+          for (int k = 0; k < kdim; ++k) {
+            const int64_t xk = STRIDED ? static_cast<int64_t>(k) * d + m : (static_cast<int64_t>(k / C) * d + m) * C + k % C;
+            const float xa = in[n * a.xwidth + g.xoff + xk];
+            val = fmaf(xa, BT ? g.w[static_cast<int64_t>(k) * ncols + col] : g.w[static_cast<int64_t>(col) * g.k + k], val);
+          }
+        }
+        val *= a.alpha;
+        out[n * a.ywidth + g.yoff + static_cast<int64_t>(col) * d + m] = val;
+      }
+    }
+  }
+}
+
+// Input adjoint on the bf16 matrix cores: gx rows = alpha gY W with a short K = O (16 KS) and many
+// columns (counts C).  A wave keeps 32 gY rows split in registers (12 KS VGPRs) and walks the columns; W
+// arrives in chunks of 64 columns, split into LDS once per block (one buffer, the next chunk's loads in
+// flight), its columns in the order even, odd so that a lane owns two neighbouring ones and stores
+// them together (256 contiguous bytes of two rows per instruction).  LinearSplit lists the launch's blocks:
+// 128 rows of one degree times `chunks` column chunks.
+// 2048 nodes, C = O = 128, counts (4, 6, 7, 6): 56 us, on fp32 MFMA 84 us (the six part products take about 29,
+// the 104 MB of gx 15; the rest is the first loads and the last partly filled round of blocks); error
+// against float64 1.6e-7, 2.0e-7 there.
+struct LinearSplit {
+  int64_t block0[ICTC_LINEAR_MAX_DEGREES + 1];   // first block of each degree
+  int splits[ICTC_LINEAR_MAX_DEGREES];           // column splits of a degree
+  int chunks, degrees;                           // column chunks per block
+};
+
+template <int KS>
+__global__ void __launch_bounds__(256, 2)
+degree_linear_input_grad_kernel(const float* __restrict__ gy, float* __restrict__ gx, const LinearArgs a,
+                                const LinearSplit sp) {
+  constexpr int K = 16 * KS, OCT = 2 * KS, PER = OCT / 4;   // octets of K; per thread and chunk
+  int z = 0;
+  const int64_t b = blockIdx.x;
+  while (z + 1 < sp.degrees && b >= sp.block0[z + 1]) ++z;
+  const DegreeGeometry g = a.g[z];
+  const int64_t t = b - sp.block0[z];
+  const int split = static_cast<int>(t % sp.splits[z]);
+  const int d = g.d, C = a.channels;
+  const int nchunks = (g.k + 63) / 64;
+  const int ch0 = split * sp.chunks, ch1 = ch0 + sp.chunks < nchunks ? ch0 + sp.chunks : nchunks;
+  __shared__ bf16x8 sB[3][OCT][64];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r = lane & 31, half = lane >> 5;
+  const int64_t row0 = (t / sp.splits[z]) * 128 + wave * 32;
+  float wv[PER][8];
+  auto fetch = [&](int ch) {   // column tid % 64, octets tid / 64 + 4 q
+    const int col = 64 * ch + (tid & 63) < g.k ? 64 * ch + (tid & 63) : g.k - 1;   // (past the end: not stored)
+    const float* __restrict__ p = g.w + static_cast<int64_t>(8 * (tid >> 6)) * g.k + col;
+#pragma unroll
+    for (int q = 0; q < PER; ++q)
+#pragma unroll
+      for (int u = 0; u < 8; ++u) wv[q][u] = p[static_cast<int64_t>(32 * q + u) * g.k];
+  };
+  auto stage = [&]() {
+    const int col = tid & 63, slot = 32 * (col & 1) + col / 2;
+#pragma unroll
+    for (int q = 0; q < PER; ++q) {
+      const Split8 s = split8(wv[q]);
+#pragma unroll
+      for (int p = 0; p < 3; ++p) sB[p][4 * q + (tid >> 6)][slot] = s.p[p];
+    }
+  };
+  fetch(ch0);
+  Split8 av[KS][1];
+  {
+    const int64_t rho = row0 + r < g.rows ? row0 + r : g.rows - 1;   // rows past the end: not stored
+    const int64_t n = rho / d;
+    const float* __restrict__ p = gy + n * a.ywidth + g.yoff + (rho - n * d) + 8 * half * d;
+#pragma unroll
+    for (int k = 0; k < KS; ++k) {
+      float v[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v[u] = p[(16 * k + u) * d];
+      av[k][0] = split8(v);
+    }
+  }
+  // byte offsets of the lane's sixteen result rows from the node of the wave's first row
+  const int64_t nbase = (row0 < g.rows ? row0 : 0) / d;
+  const int mbase = static_cast<int>((row0 < g.rows ? row0 : 0) - nbase * d);
+  float* __restrict__ obase = gx + nbase * a.xwidth + g.xoff;
+  const rsrc_t ro = make_rsrc(obase, 0x7FFFFFF0u);
+  uint32_t roff[16];
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const int q = mbase + mfma_row(i, half), dn = q / d;
+    const bool in = row0 + mfma_row(i, half) < g.rows;
+    roff[i] = in ? static_cast<uint32_t>((dn * a.xwidth + static_cast<int64_t>(q - dn * d) * C) * 4) : 0xFFFFFFF0u;
+  }
+  stage();
+  __syncthreads();
+  for (int ch = ch0; ch < ch1; ++ch) {
+    const bool more = ch + 1 < ch1;
+    if (more) fetch(ch + 1);
+    f32x16 acc[1][2];
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[0][c][i] = 0.f;
+#pragma unroll
+    for (int k = 0; k < KS; ++k) {
+      Split8 bv[2];
+#pragma unroll
+      for (int c = 0; c < 2; ++c)
+#pragma unroll
+        for (int p = 0; p < 3; ++p) bv[c].p[p] = sB[p][2 * k + half][32 * c + r];
+      mfma_split(av[k], bv, acc, acc);
+    }
+    const int col = 64 * ch + 2 * r;     // the lane's columns col, col + 1 (counts C is even)
+    const int blk = col / C;
+    const uint32_t coff = static_cast<uint32_t>(blk * d * C + (col - blk * C)) * 4u;
+    const bool redo = any_nonfinite(acc[0][0]) || any_nonfinite(acc[0][1]);   // see split_bf16.hpp: again in fp32
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      f32x2 v{acc[0][0][i], acc[0][1][i]};
+      if (redo) {
+        v = f32x2{0.f, 0.f};
+        const int64_t rho = row0 + mfma_row(i, half);
+        if (rho < g.rows && col < g.k) {
+          const int64_t n = rho / d;
+          for (int k = 0; k < K; ++k) {
+            const float y = gy[n * a.ywidth + g.yoff + static_cast<int64_t>(k) * d + (rho - n * d)];
+            const float* __restrict__ w = g.w + static_cast<int64_t>(k) * g.k + col;
+            v = f32x2{fmaf(y, w[0], v[0]), fmaf(y, w[1], v[1])};
+          }
+        }
+      }
+      v = f32x2{v[0] * a.alpha, v[1] * a.alpha};
+      const uint32_t off = roff[i] == 0xFFFFFFF0u || col >= g.k ? 0xFFFFFFF0u : roff[i] + coff;
+      __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v), ro, off, 0, 0);
+    }
+    __syncthreads();
+    if (more) {
+      stage();
+      __syncthreads();
+    }
+  }
+}
+
 int prepare(const ictc_degree_linear_desc* desc, const float* const* weights, float alpha, int64_t nodes,
             LinearArgs* a, int* live_degrees, int64_t* max_rows, int* max_cols, bool fwd) {
   if (desc == nullptr || weights == nullptr || nodes < 0) return ICTC_ERR_INVALID_ARGUMENT;
@@ -319,6 +599,30 @@ int prepare(const ictc_degree_linear_desc* desc, const float* const* weights, fl
   return ICTC_OK;
 }
 
+// Blocks of an input-adjoint launch: the column chunks per block with the fewest rounds of resident
+// blocks (two per CU), each costing its chunks and about two more for the block's own rows.
+LinearSplit input_grad_split(const LinearArgs& a, int degrees) {
+  LinearSplit best{};
+  int64_t cost = INT64_MAX;
+  for (int chunks = 1; chunks <= 64; ++chunks) {
+    LinearSplit s{};
+    s.chunks = chunks;
+    s.degrees = degrees;
+    int most = 0;
+    for (int l = 0; l < degrees; ++l) {
+      const int n = (a.g[l].k + 63) / 64;
+      s.splits[l] = n == 0 ? 1 : (n + chunks - 1) / chunks;
+      s.block0[l + 1] = s.block0[l] + (n == 0 ? 0 : (a.g[l].rows + 127) / 128 * s.splits[l]);
+      most = n > most ? n : most;
+    }
+    const int64_t slots = 2 * static_cast<int64_t>(compute_units());
+    const int64_t c = (s.block0[degrees] + slots - 1) / slots * ((chunks < most ? chunks : most) + 2);
+    if (c < cost) cost = c, best = s;
+    if (chunks >= most) break;
+  }
+  return best;
+}
+
 template <int MODE>
 int launch(const ictc_degree_linear_desc* desc, const float* in, const float* const* weights, float alpha,
            float* out, int64_t nodes, hipStream_t stream) {
@@ -344,6 +648,38 @@ int launch(const ictc_degree_linear_desc* desc, const float* in, const float* co
   const int tn = vec ? kTn : kTile;
   const dim3 grid(static_cast<unsigned>(row_tiles), static_cast<unsigned>((max_cols + tn - 1) / tn),
                   static_cast<unsigned>(degrees));
+  if (vec && MODE == kInputGrad && max_cols > 64 &&
+      (desc->out_channels == 64 || desc->out_channels == 96 || desc->out_channels == 128) &&
+      128 * a.xwidth * 4 < 0x40000000) {
+    // the register-resident rows where its 128-row blocks give every CU one
+    const LinearSplit sp = input_grad_split(a, degrees);
+    if (sp.block0[degrees] >= compute_units() && sp.block0[degrees] <= 0x7fffffff) {
+      const dim3 igrid(static_cast<unsigned>(sp.block0[degrees]));
+      if (desc->out_channels == 64)
+        hipLaunchKernelGGL(degree_linear_input_grad_kernel<4>, igrid, dim3(256), 0, stream, in, out, a, sp);
+      else if (desc->out_channels == 96)
+        hipLaunchKernelGGL(degree_linear_input_grad_kernel<6>, igrid, dim3(256), 0, stream, in, out, a, sp);
+      else
+        hipLaunchKernelGGL(degree_linear_input_grad_kernel<8>, igrid, dim3(256), 0, stream, in, out, a, sp);
+      return hipGetLastError() == hipSuccess ? ICTC_OK : ICTC_ERR_LAUNCH;
+    }
+  }
+  if constexpr (MODE != kInputGrad) {
+    // split-bf16 blocks (two per CU) where they give every CU one: fewer, larger blocks than the fp32
+    // kernel's, which keeps the smaller calls
+    const int stn = max_cols > 64 ? 128 : 64;
+    int64_t blocks = 0;
+    for (int l = 0; l < degrees; ++l) blocks += ((a.g[l].rows + kTile - 1) / kTile) * ((a.out_channels + stn - 1) / stn);
+    if (vec && blocks >= compute_units()) {
+      const dim3 sgrid(static_cast<unsigned>(row_tiles), static_cast<unsigned>((max_cols + stn - 1) / stn),
+                       static_cast<unsigned>(degrees));
+      if (stn == 128)
+        hipLaunchKernelGGL((degree_linear_split_kernel<MODE, 128>), sgrid, dim3(256), 0, stream, in, out, a);
+      else
+        hipLaunchKernelGGL((degree_linear_split_kernel<MODE, 64>), sgrid, dim3(256), 0, stream, in, out, a);
+      return hipGetLastError() == hipSuccess ? ICTC_OK : ICTC_ERR_LAUNCH;
+    }
+  }
   if (vec)
     hipLaunchKernelGGL((degree_linear_kernel<MODE, true, MODE == kForward ? 2 : 1, kTn>), grid, dim3(256), 0, stream,
                        in, out, a);
@@ -358,18 +694,19 @@ int launch(const ictc_degree_linear_desc* desc, const float* in, const float* co
 // x[n, c, m] at offset C l^2, j = c).  The rows of a degree are split into ranges (range_rows, a
 // multiple of the 32-row chunk sized so that every block of the launch is resident at once: the
 // LDS of three blocks fits a CU, and a second partial round of blocks would idle most CUs); a
-// block of kWgWaves waves computes the 128 (o) x 64 (j) partial of one range (each wave 128 /
-// kWgWaves o x 64 j, v_mfma_f32_16x16x4_f32 over 32-row chunks staged through LDS, the next
-// chunk's loads in flight
-// during the current chunk's MFMAs) and stores it into the workspace; a second kernel sums the
-// ranges in order and scales by alpha (fixed order: bit-identical run to run).  Rows past the end
-// read zeros from the buffer range check (their offsets lie past the tensors).
+// block of kWgWaves waves computes the 128 (o) x 64 (j) partial of one range (each wave 32 o x 32 j on
+// the bf16 matrix cores, fp32 operands in three parts: split_bf16.hpp) over 32-row chunks: a thread's
+// operand unit is eight rows of one column, split when the chunk is staged, the next chunk's loads in
+// flight during the current chunk's matrix instructions (one LDS buffer, two barriers per chunk).  The
+// partials go to the workspace; a second kernel sums the ranges in order and scales by alpha (fixed order:
+// bit-identical run to run).  Rows past the end read zeros from the buffer range check (their offsets lie
+// past the tensors).  2048 nodes, C = O = 128, counts (4, 6, 7, 6): 82 us with the sum, 101 us with fp32
+// MFMA; error against float64 1.7e-7, 4.4e-7 there.
 enum WgLayout { kWgIrMul = 0, kWgMulIr = 1 };
 constexpr int kWgMinRows = 256;   // shortest range (8 chunks)
-constexpr int kWgBlocksPerCu = 3;  // 51,200 B of LDS per block
+constexpr int kWgBlocksPerCu = 3;  // 36,864 B of LDS and 80 VGPRs
 constexpr int kWgO = 128, kWgJ = 64;
-constexpr int kWgWaves = 8;   // waves per block: 16 o rows x 64 j each
-constexpr int kWgPitchA = kWgO + 4, kWgPitchB = kWgJ + 4;
+constexpr int kWgWaves = 8;   // waves per block: 32 o x 32 j each
 
 struct WgDegree {
   int64_t rows;     // N d
@@ -393,7 +730,7 @@ struct WgArgs {
 };
 
 template <int LAYOUT>
-__global__ void __launch_bounds__(64 * kWgWaves)
+__global__ void __launch_bounds__(64 * kWgWaves, 6)
 degree_linear_wgrad_kernel(const float* __restrict__ gy, const float* __restrict__ x, float* __restrict__ ws,
                            const WgArgs a) {
   // XCD-contiguous block order: the column tiles of one row range (which read the same gY rows)
@@ -412,18 +749,16 @@ degree_linear_wgrad_kernel(const float* __restrict__ gy, const float* __restrict
   const int64_t r0 = static_cast<int64_t>(range) * a.range_rows;
   const int64_t r1 = r0 + a.range_rows < g.rows ? r0 + a.range_rows : g.rows;
   const int d = g.d, C = a.C, O = a.O;
-  __shared__ float sA[2][32][kWgPitchA];   // [buffer][row][o]
-  __shared__ float sB[2][32][kWgPitchB];   // [buffer][row][j]
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  __shared__ SplitTile<kWgO> sA;
+  __shared__ SplitTile<kWgJ> sB;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const rsrc_t ry = make_rsrc(gy, a.ybytes), rx = make_rsrc(x, a.xbytes);
-  // A staging: element e = tid + T i (T threads, i < NA): o = e % 128, row e / 128; o past O (or
-  // past the tile) reads o = 0 of its row: those accumulator rows are never stored.
-  constexpr int T = 64 * kWgWaves, NA = 32 * kWgO / T, NB = 32 * kWgJ / T, AR = T / kWgO, BR = T / kWgJ;
-  constexpr int OU = kWgO / 16 / kWgWaves;   // 16-row MFMA tiles per wave
-  const int ao = tid & 127, arr = tid >> 7;
+  // A units: column (o) tid % 128, rows 8 (tid / 128) ..; o past O (or past the tile) reads o = 0 of
+  // its row: those accumulator rows are never stored.  B units, the first four waves: column (j)
+  // tid % 64, rows 8 (tid / 64) ..; j past k reads column 0.
+  const bool hasb = wave < 4;   // wave-uniform
+  const int ao = tid & (kWgO - 1), aoct = tid / kWgO, bj = tid & (kWgJ - 1), boct = tid / kWgJ;
   const int aoc = o0 + ao < O ? o0 + ao : 0;
-  // B staging: element e = tid + T i (i < NB): j = e % 64, row e / 64; j past k reads column 0
-  const int bj = tid & 63, brr = tid >> 6;
   const int bjc = j0 + bj < g.k ? j0 + bj : 0;
   uint32_t bcol;   // byte offset of column bjc inside a row's degree block (m = 0)
   if constexpr (LAYOUT == kWgIrMul) {
@@ -440,80 +775,75 @@ degree_linear_wgrad_kernel(const float* __restrict__ gy, const float* __restrict
   const uint32_t yo4 = static_cast<uint32_t>(g.yoff) * 4u + static_cast<uint32_t>(aoc * d) * 4u;
   const uint32_t xo4 = static_cast<uint32_t>(g.xoff) * 4u + bcol;
   const uint32_t mstep = (LAYOUT == kWgIrMul ? static_cast<uint32_t>(C) : 1u) * 4u;
-  float ra[NA], rb[NB];
-  auto fetch = [&](int64_t c0) {
+  float ra[8], rb[8];
+  // eight rows of one column, from row c0 + first of the degree: offset n * width + base + m * step
+  // (rows past r1 belong to the next range or lie past the end: an out-of-range offset reads 0)
+  auto octet = [&](rsrc_t rs, int64_t c0, int first, uint32_t width, uint32_t base, uint32_t step, float (&v)[8]) {
     const int n0 = static_cast<int>(c0 / d), m0 = static_cast<int>(c0 - static_cast<int64_t>(n0) * d);
 #pragma unroll
-    for (int i = 0; i < NA; ++i) {
-      const int q = m0 + arr + AR * i;
+    for (int i = 0; i < 8; ++i) {
+      const int q = m0 + first + i;
       const int dn = static_cast<int>((static_cast<float>(q) + 0.5f) * inv_d), m = q - dn * d;
-      // rows past r1 belong to the next range (or past the end): an out-of-range offset reads 0
-      const uint32_t off = c0 + arr + AR * i < r1 ? static_cast<uint32_t>(n0 + dn) * yw4 + yo4 + static_cast<uint32_t>(m) * 4u
-                                                  : 0xFFFFFFF0u;
-      ra[i] = buf_load<1>(ry, off).v[0];
-    }
-#pragma unroll
-    for (int i = 0; i < NB; ++i) {
-      const int q = m0 + brr + BR * i;
-      const int dn = static_cast<int>((static_cast<float>(q) + 0.5f) * inv_d), m = q - dn * d;
-      const uint32_t off = c0 + brr + BR * i < r1 ? static_cast<uint32_t>(n0 + dn) * xw4 + xo4 + static_cast<uint32_t>(m) * mstep
-                                                  : 0xFFFFFFF0u;
-      rb[i] = buf_load<1>(rx, off).v[0];
+      const uint32_t off = static_cast<uint32_t>(n0 + dn) * width + base + static_cast<uint32_t>(m) * step;
+      v[i] = buf_load<1>(rs, c0 + first + i < r1 ? off : 0xFFFFFFF0u).v[0];
     }
   };
-  auto stage = [&](int buf) {
-#pragma unroll
-    for (int i = 0; i < NA; ++i) sA[buf][arr + AR * i][ao] = ra[i];
-#pragma unroll
-    for (int i = 0; i < NB; ++i) sB[buf][brr + BR * i][bj] = rb[i];
+  auto fetch = [&](int64_t c0) {
+    octet(ry, c0, 8 * aoct, yw4, yo4, 4u, ra);
+    if (hasb) octet(rx, c0, 8 * boct, xw4, xo4, mstep, rb);
   };
-  f32x4_t acc[OU][4] = {};
-  const int fr = lane & 15, fq = (lane >> 4) * 4;
-  auto mfma_chunk = [&](int buf) {
+  const int r = lane & 31, half = lane >> 5, o_t = (wave & 3) * 32, j_t = (wave >> 2) * 32;
+  const bool work = o0 + o_t < O && j0 + j_t < g.k;   // wave-uniform: any result to store
+  f32x16 acc[1][1], lo[1][1];
 #pragma unroll
-    for (int kg = 0; kg < 32; kg += 16) {
-      float av[OU][4], bv[4][4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-#pragma unroll
-        for (int u = 0; u < OU; ++u) av[u][j] = sA[buf][kg + fq + j][wave * 16 * OU + u * 16 + fr];
-#pragma unroll
-        for (int tt = 0; tt < 4; ++tt) bv[tt][j] = sB[buf][kg + fq + j][tt * 16 + fr];
-      }
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-#pragma unroll
-        for (int u = 0; u < OU; ++u)
-#pragma unroll
-          for (int tt = 0; tt < 4; ++tt)
-            acc[u][tt] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[u][j], bv[tt][j], acc[u][tt], 0, 0, 0);
-    }
-  };
+  for (int i = 0; i < 16; ++i) acc[0][0][i] = lo[0][0][i] = 0.f;
   fetch(r0);
-  stage(0);
-  __syncthreads();
-  int buf = 0;
   for (int64_t c0 = r0; c0 < r1; c0 += 32) {
-    const bool more = c0 + 32 < r1;
-    if (more) fetch(c0 + 32);
-    mfma_chunk(buf);
-    if (more) stage(buf ^ 1);
+    const Split8 va = split8(ra);
+#pragma unroll
+    for (int q = 0; q < 3; ++q) sA.v[q][aoct][ao] = va.p[q];
+    if (hasb) {
+      const Split8 vb = split8(rb);
+#pragma unroll
+      for (int q = 0; q < 3; ++q) sB.v[q][boct][bj] = vb.p[q];
+    }
     __syncthreads();
-    buf ^= 1;
+    if (c0 + 32 < r1) fetch(c0 + 32);
+    if (work) {
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        Split8 av[1], bv[1];
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+          av[0].p[q] = sA.v[q][2 * k + half][o_t + r];
+          bv[0].p[q] = sB.v[q][2 * k + half][j_t + r];
+        }
+        mfma_split(av, bv, acc, lo);
+      }
+    }
+    __syncthreads();
   }
   float* __restrict__ part = ws + g.ws0 + static_cast<int64_t>(range) * O * g.k;
+  const int j = j0 + j_t + r;
 #pragma unroll
-  for (int u = 0; u < OU; ++u)
+  for (int i = 0; i < 16; ++i) acc[0][0][i] += lo[0][0][i];
+  const bool redo = any_nonfinite(acc[0][0]);   // see split_bf16.hpp: these results again in fp32
 #pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const int o = o0 + wave * 16 * OU + u * 16 + 4 * (lane >> 4) + v;
-      if (o >= O) continue;
-#pragma unroll
-      for (int tt = 0; tt < 4; ++tt) {
-        const int j = j0 + tt * 16 + fr;
-        if (j < g.k) part[static_cast<int64_t>(o) * g.k + j] = acc[u][tt][v];
+  for (int i = 0; i < 16; ++i) {
+    const int o = o0 + o_t + mfma_row(i, half);
+    if (o >= O || j >= g.k) continue;
+    float v = acc[0][0][i];
+    if (redo) {
+      v = 0.f;
+      for (int64_t rho = r0; rho < r1; ++rho) {
+        const int64_t n = rho / d, m = rho - n * d;
+        const int64_t xj = LAYOUT == kWgIrMul ? (static_cast<int64_t>(j / C) * d + m) * C + j % C
+                                              : static_cast<int64_t>(j) * d + m;
+        v = fmaf(gy[n * a.ywidth + g.yoff + static_cast<int64_t>(o) * d + m], x[n * a.xwidth + g.xoff + xj], v);
       }
     }
+    part[static_cast<int64_t>(o) * g.k + j] = v;
+  }
 }
 
 // gW_l = alpha * the sum of the degree's range partials, in range order (one thread per entry).

@@ -1,4 +1,4 @@
-"""Per-degree channel linear on the fp32-MFMA kernels of ``csrc/linear_api.hip``: the
+"""Per-degree channel linear on the matrix-core kernels of ``csrc/linear_api.hip``: the
 path-preserving message linear of the MACE interaction (reference
 ``mace_ictc/models/pure_cartesian_ictd_fix.py:629-661``), read straight from the message
 kernels' packed ir_mul output and written in the mul_ir node layout.

@@ -773,8 +773,16 @@ int launch_msg_forward_tangent(const ictc_tp_desc& d, const float* x, const floa
 // t = (tx, tY, tg) with dout fixed (the mixed second derivatives): tw_I = sum_J tY_{l2^2 + J} U_p[I][J],
 //   dg_p = sum_I (tx_I w_I + x_I tw_I),  dxe_I += g_p tw_I + tg_p w_I,
 //   dY_{l2^2 + J} += sum_I (tx_I g_p + x_I tg_p) U_p[I][J].
-// One block per (receiver, 64-channel chunk); path k's U block is built by wave k mod 4, then every
-// wave walks every fourth edge of the receiver.  dY partials [edges, chunks, NY]: group launches run
+// One block per (receiver, 64-channel chunk), of msg_grad_waves waves; path k's U block is built by wave
+// k mod 4 (mod 8 in the larger blocks), then each wave walks its share of the receiver's edges.
+// Bound by HBM: the gates in, their gradient and dxe out (3.3 GB for C = 128, lmax 3, 106,304 edges: 680 us at
+// a large copy's 4.9 TB/s).  No wait in the edge loop may take in more than it needs: indices and
+// harmonics come by vector loads (scalar loads share their counter with the LDS reads), the next
+// edge's loads are in flight throughout, and the next U row's reads behind the current row's products, with
+// no branch in between (WY, ACC are template parameters).  At that size the four launches take
+// 0.95 ms, without the harmonics gradient 0.75 ms, the tangent without it 1.03 ms (before: scalar index and harmonics
+// loads in the loop, 4 waves per block: 1.05, 0.83 and 1.10 ms); 5,219 edges over 256 receivers, C = 64,
+// lmax 2: 26 us (49 us); outputs bit-identical.  dY partials [edges, chunks, NY]: group launches run
 // in order on one stream; the first writes each (edge, chunk) slot, later groups add to it (a fixed
 // order; the caller sums the chunk axis).
 struct NodeU {
@@ -799,17 +807,57 @@ struct NodeUOf {
   static constexpr NodeU tab = make_node_u<LIN, LE, LOUT, L1>();
 };
 
-// Resident waves per SIMD the compiler is held to for an edge-gradient launch of an lmax-3 set
-// (register budget 512 / waves), where its LDS allows more waves than its unconstrained register
-// allocation: input degree 2 first order at 4 (128 VGPRs; its 39.7 KB table allows 4 blocks per
-// CU, 130 VGPRs would allow 3), input degree 3 tangent at 3 (168 VGPRs; 173 allowed 2, its 50 KB
-// table 3).
-constexpr int msg_edge_grad_waves(int lin, int l1, bool jvp) {
-  return lin < 3 ? 1 : l1 == 2 && !jvp ? 4 : l1 == 3 && jvp ? 3 : 1;
+// The compiler forms v before this point.
+__device__ __forceinline__ void pin(float& v) { asm volatile("" : "+v"(v)); }
+
+// The edges of one wave of a receiver's block: wave w takes the slots s0 + w, s0 + w + waves, ... of the
+// receiver's CSR range.  The indices and sources of 64 of them are loaded at once, one per lane, and
+// read back lane by lane, so that an edge has no chain of index loads (perm -> src -> rows) in front of
+// its own loads and no scalar load in flight beside its LDS reads (both share one counter, and scalar
+// loads return out of order, so a wait for either is a wait for all).
+struct WaveEdges {
+  const int64_t *perm, *src;
+  int64_t s1, slot;   // end of the range; next slot
+  int waves, lane, at;
+  uint32_t elo, ehi, sl;
+  __device__ __forceinline__ WaveEdges(const int64_t* perm_, const int64_t* src_, int64_t s0, int64_t s1_, int wave,
+                                       int waves_, int lane_)
+      : perm(perm_), src(src_), s1(s1_), slot(s0 + wave), waves(waves_), lane(lane_), at(kWave - 1), elo(0), ehi(0),
+        sl(0) {}
+  __device__ __forceinline__ bool more() const { return slot < s1; }
+  __device__ __forceinline__ int64_t next() {   // more() only
+    at = (at + 1) & (kWave - 1);
+    if (at == 0) {   // wave-uniform
+      int64_t s = slot + static_cast<int64_t>(lane) * waves;
+      s = s < s1 ? s : s1 - 1;
+      const int64_t e = perm ? perm[s] : s;
+      elo = static_cast<uint32_t>(e);
+      ehi = static_cast<uint32_t>(static_cast<uint64_t>(e) >> 32);
+      sl = static_cast<uint32_t>(src[e]);
+    }
+    slot += waves;
+    const uint32_t lo = __builtin_amdgcn_readlane(elo, at), hi = __builtin_amdgcn_readlane(ehi, at);
+    return static_cast<int64_t>(static_cast<uint64_t>(hi) << 32 | lo);
+  }
+  __device__ __forceinline__ uint32_t source() const { return __builtin_amdgcn_readlane(sl, at); }   // of next()'s
+};
+
+constexpr int kMsgGradWaves = 16;   // most waves of a block (128 VGPRs)
+
+// Waves per block, each walking its share of the receiver's edges beside one U table.  A block's LDS (50 KB
+// for input degree 3 at lmax 3) allows three blocks per CU, so 4 waves per block leave 3 waves per SIMD
+// to hide an edge's loads; 8 give 4 to 5.  Measured with 4, 8 and 16 waves (us; first order with
+// harmonics gradient / tangent without): C = 128, lmax 3, 106,304 edges over 2,048 receivers 1020 / 1084,
+// 987 / 1044, 1067 / 1096; C = 64, lmax 2, 852,297 edges over 16,384 receivers 1514 / 1876, 1618 / 1840, 1976 /
+// 1964 (with the harmonics gradient the channel sums' exchanges bound the denser waves); a launch of
+// at most two blocks per CU, C = 64, lmax 2, 5,219 edges over 256 receivers 49 / 46, 33 / 31, 26 / 26.
+inline int msg_grad_waves(int lin, bool harmonics, int64_t blocks) {
+  if (blocks <= 2 * static_cast<int64_t>(compute_units())) return kMsgGradWaves;
+  return lin >= 3 || !harmonics ? 8 : 4;
 }
 
-template <int LIN, int LE, int LOUT, int L1, bool JVP, bool ACC = false>
-__global__ void __launch_bounds__(kMsgBlock) __attribute__((amdgpu_waves_per_eu(msg_edge_grad_waves(LIN, L1, JVP))))
+template <int LIN, int LE, int LOUT, int L1, bool JVP, bool ACC, bool WY>
+__global__ void __launch_bounds__(kWave * kMsgGradWaves)
 msg_edge_grad_degree_kernel(const float* __restrict__ x, const float* __restrict__ y, const float* __restrict__ g,
                           const MsgTangent t, const float* __restrict__ go, const int64_t* __restrict__ src,
                           const int64_t* __restrict__ rowptr, const int64_t* __restrict__ perm,
@@ -826,6 +874,7 @@ msg_edge_grad_degree_kernel(const float* __restrict__ x, const float* __restrict
   __shared__ float sU[NU * kWave];
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int waves = __builtin_amdgcn_readfirstlane(blockDim.x / kWave);
   const uint32_t item = xcd_block(blockIdx.x, gridDim.x);   // receivers contiguous per XCD
   const int64_t node = static_cast<int64_t>(item) / nchunks;
   const int chunk = static_cast<int>(item - node * nchunks);
@@ -839,7 +888,7 @@ msg_edge_grad_degree_kernel(const float* __restrict__ x, const float* __restrict
     const rsrc_t ron = make_rsrc(go + node * NOCF * C, NOCF * row);
     static_for<0, NPG>([&](auto Q) {
       constexpr int k = Q;
-      if (wave == k % kMsgWaves) {   // wave-uniform
+      if (wave == (waves >= 8 ? k & 7 : k & 3)) {   // wave-uniform
         constexpr int p = GT.path[k];
         constexpr int l2 = PS::tab.l2[p], l3 = PS::tab.l3[p];
         constexpr int nj = 2 * l2 + 1, no = 2 * l3 + 1, oo = GT.out[k], uo = UT.off[k];
@@ -866,33 +915,32 @@ msg_edge_grad_degree_kernel(const float* __restrict__ x, const float* __restrict
   }
   __syncthreads();
   const uint32_t xbytes = static_cast<uint32_t>(nodes_src * NX * row);
-  const bool xdep = JVP || dg != nullptr || dyp != nullptr;   // the plain dxe needs no x
+  const bool xdep = JVP || WY || dg != nullptr;   // the plain dxe needs no x
   const rsrc_t rx[2] = {make_rsrc(xdep ? x : nullptr, xbytes), make_rsrc(JVP ? t.x : nullptr, xbytes)};
   const float* gs[2] = {g, t.g};
   const float* ys[2] = {y, t.y};
-  const bool wy = dyp != nullptr;
   using WS = WaveSums<NY>;
   const int wj = WS::index(lane);   // the harmonic whose channel sum this lane ends up holding
-  const bool wown = wy && WS::owner(lane) && wj < NY;
+  const bool wown = WY && WS::owner(lane) && wj < NY;
   const int wjc = wj < NY ? wj : NY - 1;
-  // One edge's inputs: its harmonics rows (wave-uniform loads), the source features of degree l1,
-  // the group's gates and the harmonics partial that earlier degree launches left in the slot.
+  const int yj = lane < NY ? lane : NY - 1;
+  // One edge's inputs: its harmonics rows (one value per lane), the source features of degree l1, the
+  // group's gates and the harmonics partial that earlier degree launches left in the slot.  All vector
+  // loads: a scalar load in flight would make the first LDS wait below wait for it too.
   struct EdgeIn {
-    float yv[NT][NY];
+    float yl[NT];
     float xr[NT][NI];
     float gv[NT][NPG];
     float dgp[ACC ? NPG : 1];   // ACC: the gate gradients already in dg (this pass adds to them)
     float prev;
   };
-  auto fetch = [&](int64_t e, int64_t s, EdgeIn& in) {
+  auto fetch = [&](int64_t e, uint32_t s, EdgeIn& in) {
 #pragma unroll
-    for (int q = 0; q < NT; ++q)
-#pragma unroll
-      for (int j = 0; j < NY; ++j) in.yv[q][j] = ys[q][e * NY + j];
+    for (int q = 0; q < NT; ++q) in.yl[q] = ys[q][e * NY + yj];
     // Lanes past C get a voffset beyond the descriptor's range (xdead), so the hardware returns
     // 0: a select on the loaded value instead would make the wave wait for this (prefetched)
     // gather before computing the current edge.
-    const uint32_t xoff = (static_cast<uint32_t>(s) * NX * row + vc) | xdead;
+    const uint32_t xoff = (s * NX * row + vc) | xdead;
 #pragma unroll
     for (int q = 0; q < NT; ++q)
 #pragma unroll
@@ -908,136 +956,121 @@ msg_edge_grad_degree_kernel(const float* __restrict__ x, const float* __restrict
 #pragma unroll
       for (int k = 0; k < NPG; ++k) in.dgp[k] = buf_load_vs(rdg, vc, GT.path[k] * row);
     }
-    in.prev = (wy && !first) ? dyp[(e * nchunks + chunk) * NY + wjc] : 0.f;
+    in.prev = (WY && !first) ? dyp[(e * nchunks + chunk) * NY + wjc] : 0.f;
   };
+  // One row I of a path's U block: nj entries per lane.
+  auto load_row = [&](auto ROW, float* u) {
+    constexpr int k = ROW / NI, i = ROW % NI;
+    constexpr int nj = 2 * PS::tab.l2[GT.path[k]] + 1;
+    const float* up = opaque_lds_row(sU);   // keeps the reads between the barriers around them
+#pragma unroll
+    for (int j = 0; j < nj; ++j) u[j] = up[(UT.off[k] + i * nj + j) * kWave + lane];
+  };
+  // One edge's adjoints, the U rows of all paths in one sequence: a row's reads are issued before the
+  // products of the row ahead of it.
   auto compute = [&](int64_t e, const EdgeIn& in) {
-    const rsrc_t rdg = make_rsrc(dg ? dg + e * NP * C : nullptr, NP * row);
-    float dyl[NY], dxl[NI];
+    float yv[NT][NY], dyl[NY], dxl[NI], dgv = 0.f, vp[7], ub[2][7];
+#pragma unroll
+    for (int n = 0; n < NT; ++n)
+#pragma unroll
+      for (int j = 0; j < NY; ++j)
+        yv[n][j] = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, in.yl[n]), j));
 #pragma unroll
     for (int j = 0; j < NY; ++j) dyl[j] = 0.f;
 #pragma unroll
     for (int m = 0; m < NI; ++m) dxl[m] = 0.f;
-    static_for<0, NPG>([&](auto Q) {
-      constexpr int k = Q;
+    load_row(Int<0>{}, ub[0]);
+    static_for<0, NPG * NI>([&](auto ROW) {
+      constexpr int k = ROW / NI, i = ROW % NI;
       constexpr int p = GT.path[k];
       constexpr int l2 = PS::tab.l2[p];
-      constexpr int nj = 2 * l2 + 1, uo = UT.off[k];
-      const float* up = opaque_lds_row(sU + uo * kWave);
+      constexpr int nj = 2 * l2 + 1, y0 = l2 * l2;
+      if constexpr (ROW + 1 < NPG * NI) load_row(Int<ROW + 1>{}, ub[(ROW + 1) & 1]);
       __builtin_amdgcn_sched_barrier(0);
-      float w[NI], tw[NI];
+      const float* u = ub[ROW & 1];
+      if constexpr (i == 0) {
+        dgv = 0.f;
 #pragma unroll
-      for (int i = 0; i < NI; ++i) w[i] = tw[i] = 0.f;
-      float dgv = 0.f;
+        for (int j = 0; j < nj; ++j) vp[j] = 0.f;
+      }
+      float w = 0.f, tw = 0.f;
       if constexpr (JVP) {
         // harmonics partials from xg_I = tx_I g_p + x_I tg_p
-        auto contract = [&](auto WY) {
-          float xg[NI], part[nj];
-          if constexpr (WY) {
+        const float xg = fmaf(in.xr[1][i], in.gv[0][k], in.xr[0][i] * in.gv[1][k]);
 #pragma unroll
-            for (int i = 0; i < NI; ++i) xg[i] = fmaf(in.xr[1][i], in.gv[0][k], in.xr[0][i] * in.gv[1][k]);
-#pragma unroll
-            for (int j = 0; j < nj; ++j) part[j] = 0.f;
-          }
-          static_for<0, NI>([&](auto I) {
-            __builtin_amdgcn_sched_barrier(0);   // one row of U in registers at a time
-            static_for<0, nj>([&](auto J) {
-              const float u = up[(I * nj + J) * kWave + lane];
-              w[I] = fmaf(in.yv[0][l2 * l2 + J], u, w[I]);
-              tw[I] = fmaf(in.yv[1][l2 * l2 + J], u, tw[I]);
-              if constexpr (WY) part[J] = fmaf(xg[I], u, part[J]);
-            });
-          });
-          if constexpr (WY) {
-#pragma unroll
-            for (int j = 0; j < nj; ++j) dyl[l2 * l2 + j] += part[j];
-          }
-        };
-        if (wy)
-          contract(Int<1>{});
-        else
-          contract(Int<0>{});
-#pragma unroll
-        for (int i = 0; i < NI; ++i) {
-          dgv = fmaf(in.xr[1][i], w[i], dgv);
-          dgv = fmaf(in.xr[0][i], tw[i], dgv);
-          dxl[i] = fmaf(in.gv[0][k], tw[i], dxl[i]);
-          dxl[i] = fmaf(in.gv[1][k], w[i], dxl[i]);
+        for (int j = 0; j < nj; ++j) {
+          w = fmaf(yv[0][y0 + j], u[j], w);
+          tw = fmaf(yv[1][y0 + j], u[j], tw);
+          if constexpr (WY) vp[j] = fmaf(xg, u[j], vp[j]);
         }
+        dgv = fmaf(in.xr[1][i], w, dgv);
+        dgv = fmaf(in.xr[0][i], tw, dgv);
+        dxl[i] = fmaf(in.gv[0][k], tw, dxl[i]);
+        dxl[i] = fmaf(in.gv[1][k], w, dxl[i]);
       } else {
-        // with v_J = sum_I x_I U[I][J]: dg_p = sum_J Y_J v_J and the partials are g_p v_J
-        auto contract = [&](auto WY) {
-          float v[nj];
-          if constexpr (WY) {
 #pragma unroll
-            for (int j = 0; j < nj; ++j) v[j] = 0.f;
-          }
-          static_for<0, NI>([&](auto I) {
-            __builtin_amdgcn_sched_barrier(0);   // one row of U in registers at a time
-            static_for<0, nj>([&](auto J) {
-              const float u = up[(I * nj + J) * kWave + lane];
-              w[I] = fmaf(in.yv[0][l2 * l2 + J], u, w[I]);
-              if constexpr (WY) v[J] = fmaf(in.xr[0][I], u, v[J]);
-            });
-          });
-          if constexpr (WY) {
-#pragma unroll
-            for (int j = 0; j < nj; ++j) {
-              dgv = fmaf(in.yv[0][l2 * l2 + j], v[j], dgv);
-              dyl[l2 * l2 + j] = fmaf(in.gv[0][k], v[j], dyl[l2 * l2 + j]);
-            }
-          } else {
-#pragma unroll
-            for (int i = 0; i < NI; ++i) dgv = fmaf(in.xr[0][i], w[i], dgv);
-          }
-        };
-        if (wy)
-          contract(Int<1>{});
-        else
-          contract(Int<0>{});
-#pragma unroll
-        for (int i = 0; i < NI; ++i) dxl[i] = fmaf(in.gv[0][k], w[i], dxl[i]);
+        for (int j = 0; j < nj; ++j) {
+          w = fmaf(yv[0][y0 + j], u[j], w);
+          if constexpr (WY) vp[j] = fmaf(in.xr[0][i], u[j], vp[j]);
+        }
+        if constexpr (!WY) dgv = fmaf(in.xr[0][i], w, dgv);
+        dxl[i] = fmaf(in.gv[0][k], w, dxl[i]);
       }
-      if constexpr (ACC) dgv += in.dgp[k];
-      buf_store_lane(rdg, live, vc + p * row, dgv);   // null dg: empty descriptor
+      if constexpr (i == NI - 1) {
+        if constexpr (WY) {
+#pragma unroll
+          for (int j = 0; j < nj; ++j) {
+            if constexpr (JVP) {
+              dyl[y0 + j] += vp[j];
+            } else {   // with v_J = sum_I x_I U[I][J]: dg_p = sum_J Y_J v_J and the partials are g_p v_J
+              dgv = fmaf(yv[0][y0 + j], vp[j], dgv);
+              dyl[y0 + j] = fmaf(in.gv[0][k], vp[j], dyl[y0 + j]);
+            }
+          }
+        }
+        const rsrc_t rdg = make_rsrc(dg ? dg + e * NP * C : nullptr, NP * row);
+        if constexpr (ACC) dgv += in.dgp[k];
+        buf_store_lane(rdg, live, vc + p * row, dgv);   // null dg: empty descriptor
+      }
+      // the row's sums are formed here, not where the path or the edge needs them
+      if constexpr (WY) {
+#pragma unroll
+        for (int j = 0; j < nj; ++j) pin(i < NI - 1 ? vp[j] : dyl[y0 + j]);
+      }
+      pin(dgv);
+      pin(dxl[i]);
+      __builtin_amdgcn_sched_barrier(0);
     });
     if (dxe != nullptr) {
       const rsrc_t rde = make_rsrc(dxe + e * NX * C, NX * row);
 #pragma unroll
       for (int m = 0; m < NI; ++m) buf_store_lane(rde, live, vc + (L1 * L1 + m) * row, dxl[m]);
     }
-    if (wy) {   // channel sums of the NY partials, one transposing butterfly
+    if constexpr (WY) {   // channel sums of the NY partials, one transposing butterfly
       const float tot = WS::reduce(dyl, lane);
       if (wown) dyp[(e * nchunks + chunk) * NY + wj] = in.prev + tot;
     }
   };
-  // Software pipeline over the receiver's edges: the next edge's index and source (and, where the
-  // registers allow, its loads) are requested before the current edge is computed and stored.
-  constexpr bool kPrefetch = !JVP || L1 == 0;
-  const int64_t s0 = rowptr[node], s1 = rowptr[node + 1];
-  int64_t slot = s0 + wave;
-  if (slot < s1) {
-    int64_t e = perm ? perm[slot] : slot;
+  // Software pipeline over the wave's edges: an edge's loads are issued before the edge ahead of it is
+  // computed and stored.
+  WaveEdges list(perm, src, rowptr[node], rowptr[node + 1], wave, waves, lane);
+  if (list.more()) {
     EdgeIn cur;
-    fetch(e, src[e], cur);
+    int64_t e = list.next();
+    fetch(e, list.source(), cur);
 #pragma clang loop unroll(disable)
     for (;;) {
-      const int64_t nslot = slot + kMsgWaves;
-      const bool more = nslot < s1;
-      int64_t ne = e, ns = 0;
+      const bool more = list.more();
+      int64_t ne = e;
       EdgeIn nxt;
       if (more) {
-        ne = perm ? perm[nslot] : nslot;
-        ns = src[ne];
-        if constexpr (kPrefetch) fetch(ne, ns, nxt);
+        ne = list.next();
+        fetch(ne, list.source(), nxt);
       }
       compute(e, cur);
       if (!more) break;
-      slot = nslot;
       e = ne;
-      if constexpr (kPrefetch)
-        cur = nxt;
-      else
-        fetch(e, ns, cur);
+      cur = nxt;
     }
   }
 }
@@ -1068,20 +1101,22 @@ int launch_msg_edge_grad_degrees(const ictc_tp_desc& d, const float* x, const fl
                                  int64_t nodes_dst, hipStream_t stream, bool accumulate = false) {
   const int nchunks = (d.channels + kWave - 1) / kWave;
   const dim3 grid(static_cast<unsigned>(nodes_dst * nchunks));   // one block per (receiver, chunk)
+  const int waves = msg_grad_waves(LIN, dyp != nullptr, nodes_dst * nchunks);
   int first = 1;
   auto one = [&](auto deg) {
     constexpr int L1 = decltype(deg)::value;
     if constexpr (DegreeGroupOf<LIN, LE, LOUT, L1>::tab.np > 0) {
-      if constexpr (!JVP) {
-        if (accumulate) {
-          hipLaunchKernelGGL((msg_edge_grad_degree_kernel<LIN, LE, LOUT, L1, false, true>), grid, dim3(kMsgBlock), 0,
-                             stream, x, y, g, t, go, src, rowptr, perm, dyp, dg, dxe, d, nodes_src, nchunks, first);
-          first = 0;
-          return;
-        }
-      }
-      hipLaunchKernelGGL((msg_edge_grad_degree_kernel<LIN, LE, LOUT, L1, JVP>), grid, dim3(kMsgBlock), 0, stream, x,
-                         y, g, t, go, src, rowptr, perm, dyp, dg, dxe, d, nodes_src, nchunks, first);
+      auto launch = [&](auto ACC, auto WY) {
+        hipLaunchKernelGGL((msg_edge_grad_degree_kernel<LIN, LE, LOUT, L1, JVP, decltype(ACC)::value != 0,
+                                                        decltype(WY)::value != 0>),
+                           grid, dim3(kWave * waves), 0, stream, x, y, g, t, go, src, rowptr, perm, dyp, dg, dxe, d,
+                           nodes_src, nchunks, first);
+      };
+      const bool wy = dyp != nullptr;
+      if (!JVP && accumulate)
+        wy ? launch(Int<!JVP>{}, Int<1>{}) : launch(Int<!JVP>{}, Int<0>{});
+      else
+        wy ? launch(Int<0>{}, Int<1>{}) : launch(Int<0>{}, Int<0>{});
       first = 0;
     }
   };

@@ -28,6 +28,32 @@ dim3 wave_blocks(int64_t atoms) { return dim3(static_cast<unsigned>((atoms + kGr
 
 extern "C" {
 
+int ictc_hip_radius_graph_bins(const ictc_cell_grid* grid, const double* fractional, int64_t atoms,
+                               int64_t* wrap_images, double* wrapped, int32_t* atom_bins, int64_t* bin_counts,
+                               int32_t* places, hipStream_t stream) {
+  const int st = ictc::grid_status(grid, fractional, atom_bins, bin_counts, bin_counts, 0);
+  if (st != ICTC_OK) return st;
+  if (atoms < 0) return ICTC_ERR_INVALID_ARGUMENT;
+  if (atoms == 0) return ICTC_OK;
+  if (!atom_bins || !bin_counts || !places || (fractional && (!wrap_images || !wrapped))) return ICTC_ERR_INVALID_ARGUMENT;
+  if (fractional && !(grid->periodic[0] && grid->periodic[1] && grid->periodic[2])) return ICTC_ERR_INVALID_ARGUMENT;
+  hipLaunchKernelGGL(ictc::radius_bins_kernel, ictc::grid_blocks(atoms), dim3(256), 0, stream, fractional, atoms, *grid,
+                     wrap_images, wrapped, atom_bins, bin_counts, places);
+  return hipGetLastError() == hipSuccess ? ICTC_OK : ICTC_ERR_LAUNCH;
+}
+
+int ictc_hip_radius_graph_bin_atoms(const ictc_cell_grid* grid, const int32_t* atom_bins, const int32_t* places,
+                                    const int64_t* bin_start, int64_t atoms, int64_t* bin_atoms, hipStream_t stream) {
+  const int st = ictc::grid_status(grid, nullptr, atom_bins, bin_start, bin_atoms, 0);
+  if (st != ICTC_OK) return st;
+  if (atoms < 0) return ICTC_ERR_INVALID_ARGUMENT;
+  if (atoms == 0) return ICTC_OK;
+  if (!atom_bins || !places || !bin_start || !bin_atoms) return ICTC_ERR_INVALID_ARGUMENT;
+  hipLaunchKernelGGL(ictc::bin_atoms_kernel, ictc::grid_blocks(atoms), dim3(256), 0, stream, atom_bins, places, bin_start,
+                     atoms, *grid, bin_atoms);
+  return hipGetLastError() == hipSuccess ? ICTC_OK : ICTC_ERR_LAUNCH;
+}
+
 int ictc_hip_radius_graph_count(const ictc_cell_grid* grid, const double* wrapped_positions,
                                 const int32_t* atom_bins, const int64_t* bin_start, const int64_t* bin_atoms,
                                 int64_t atoms, int64_t* counts, hipStream_t stream) {

@@ -99,7 +99,7 @@ const char* ictc_hip_status_string(int status) {
   }
 }
 
-int ictc_hip_abi_version(void) { return 24; }
+int ictc_hip_abi_version(void) { return 25; }
 
 int ictc_hip_tp_slot_count(int input_lmax, int edge_lmax, int output_lmax) {
   constexpr int L = ictc::kGenericMaxL;

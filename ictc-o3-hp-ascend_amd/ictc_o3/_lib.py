@@ -15,7 +15,7 @@ import torch  # noqa: F401  (must precede CDLL, see module docstring)
 
 MAX_PATHS = 128
 LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "lib", "libictc_hip.so")
-ABI_VERSION = 24
+ABI_VERSION = 25
 
 
 class TpDesc(ctypes.Structure):
@@ -123,6 +123,8 @@ _SIGNATURES = {
     "ictc_hip_gates_weight_grad": (ctypes.c_int, [_P, _I64, _P, _P, _I64, _P, _I64, _I64, _I64, _I64, _P]),
     "ictc_hip_sgemm": (ctypes.c_int, [ctypes.c_int, ctypes.c_int, _I64, _I64, _I64, ctypes.c_float, _P, _I64, _P,
                                       _I64, ctypes.c_float, _P, _I64, _P]),
+    "ictc_hip_radius_graph_bins": (ctypes.c_int, [ctypes.POINTER(CellGrid), _P, _I64, _P, _P, _P, _P, _P, _P]),
+    "ictc_hip_radius_graph_bin_atoms": (ctypes.c_int, [ctypes.POINTER(CellGrid), _P, _P, _P, _I64, _P, _P]),
     "ictc_hip_radius_graph_count": (ctypes.c_int, [ctypes.POINTER(CellGrid), _P, _P, _P, _P, _I64, _P, _P]),
     "ictc_hip_radius_graph_fill": (ctypes.c_int, [ctypes.POINTER(CellGrid), _P, _P, _P, _P, _I64, _P, _P, _P,
                                                   _P]),

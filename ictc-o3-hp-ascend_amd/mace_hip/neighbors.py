@@ -14,7 +14,7 @@ resolved deterministically.  ``saturated`` reports whether any receiver has at l
 Host steps (device tensors): fractional coordinates, wrap along periodic axes, bins at
 least one cutoff wide along every face normal (fewer bins and a wider reach when the cell
 is narrower than the cutoff, so every image is enumerated exactly once), atoms grouped by
-bin, count pass (one wave per receiver), exclusive scan, one device-to-host read of the edge
+bin (a counting sort: ``ictc_hip_radius_graph_bins`` / ``_bin_atoms``), count pass (one wave per receiver), exclusive scan, one device-to-host read of the edge
 count and the longest row, then the sorted fill: one wave per receiver writes its row already
 ordered by (src, shift), with dst and the float64 shifts.  A row longer than the kernel's LDS
 key capacity (1,024 edges) takes the unsorted fill and two stable sorts here instead.
@@ -88,13 +88,12 @@ def radius_graph_pbc_gpu(pos: torch.Tensor, r: float, cell: torch.Tensor, max_nu
         return empty + (False,) if return_saturation else empty
     cell_cpu = cell_mat.detach().double().cpu()
     heights = _face_heights(cell_cpu)
-    c64 = cell_cpu.to(dev)
-    frac = pos.double() @ torch.linalg.inv(cell_cpu).to(dev)
-    if all(flags):
+    c64, inverse = torch.stack((cell_cpu, torch.linalg.inv(cell_cpu))).to(dev).unbind(0)
+    frac = pos.double() @ inverse
+    wrapped = all(flags)
+    if wrapped:
         # every axis wraps into [0, 1): the binned region is the cell itself, known on the host
-        n0 = torch.floor(frac)
-        fw = frac - n0
-        lo, span, span_host = None, None, [1.0, 1.0, 1.0]
+        span_host = [1.0, 1.0, 1.0]
     else:
         periodic = torch.tensor(flags, device=dev)
         n0 = torch.where(periodic, torch.floor(frac), torch.zeros_like(frac))
@@ -112,17 +111,6 @@ def radius_graph_pbc_gpu(pos: torch.Tensor, r: float, cell: torch.Tensor, max_nu
     for a in range(3):
         k = max(1, math.ceil(r / (extents[a] / bins[a])))         # bins of width extent / bins
         reach.append(min(k, bins[a] - 1) if not flags[a] else k)
-    bins_t = torch.tensor(bins, dtype=torch.float64, device=dev)
-    abin = torch.floor((fw if lo is None else (fw - lo) / span) * bins_t).clamp(min=0)
-    abin = torch.minimum(abin, bins_t - 1).to(torch.int32).contiguous()
-    wpos = (fw @ c64).contiguous()
-    ab = abin.to(torch.int64)
-    bin_id = (ab[:, 0] * bins[1] + ab[:, 1]) * bins[2] + ab[:, 2]
-    nbins = bins[0] * bins[1] * bins[2]
-    bin_atoms = torch.sort(bin_id, stable=True).indices.contiguous()
-    bin_start = torch.zeros(nbins + 1, dtype=torch.int64, device=dev)
-    torch.cumsum(torch.bincount(bin_id, minlength=nbins), 0, out=bin_start[1:])
-
     grid = _lib.CellGrid()
     for i, v in enumerate(cell_cpu.reshape(-1).tolist()):
         grid.cell[i] = v
@@ -130,6 +118,27 @@ def radius_graph_pbc_gpu(pos: torch.Tensor, r: float, cell: torch.Tensor, max_nu
     for a in range(3):
         grid.bins[a], grid.reach[a], grid.periodic[a] = bins[a], reach[a], int(flags[a])
     lib, stream = _lib.lib(), _lib.stream_of(dev)
+    if wrapped:   # wrap images, wrapped coordinates and bins by the kernel that counts the bins
+        frac = frac.contiguous()
+        n0i = torch.empty(n, 3, dtype=torch.int64, device=dev)
+        fw = torch.empty_like(frac)
+        abin = torch.empty(n, 3, dtype=torch.int32, device=dev)
+    else:
+        bins_t = torch.tensor(bins, dtype=torch.float64, device=dev)
+        abin = torch.floor((fw - lo) / span * bins_t).clamp(min=0)
+        abin = torch.minimum(abin, bins_t - 1).to(torch.int32).contiguous()
+        n0i = n0.to(torch.int64).contiguous()
+    bin_start = torch.zeros(bins[0] * bins[1] * bins[2] + 1, dtype=torch.int64, device=dev)
+    places = torch.empty(n, dtype=torch.int32, device=dev)
+    bin_atoms = torch.empty(n, dtype=torch.int64, device=dev)
+    _lib.check(lib.ictc_hip_radius_graph_bins(ctypes.byref(grid), frac.data_ptr() if wrapped else None, n,
+                                              n0i.data_ptr(), fw.data_ptr(), abin.data_ptr(), bin_start.data_ptr(),
+                                              places.data_ptr(), stream), "ictc_hip_radius_graph_bins")
+    bin_start = torch.cumsum(bin_start, 0)
+    _lib.check(lib.ictc_hip_radius_graph_bin_atoms(ctypes.byref(grid), abin.data_ptr(), places.data_ptr(),
+                                                   bin_start.data_ptr(), n, bin_atoms.data_ptr(), stream),
+               "ictc_hip_radius_graph_bin_atoms")
+    wpos = (fw @ c64).contiguous()
     args = (ctypes.byref(grid), wpos.data_ptr(), abin.data_ptr(), bin_start.data_ptr(), bin_atoms.data_ptr(), n)
     counts = torch.empty(n, dtype=torch.int64, device=dev)
     _lib.check(lib.ictc_hip_radius_graph_count(*args, counts.data_ptr(), stream), "ictc_hip_radius_graph_count")
@@ -139,7 +148,6 @@ def radius_graph_pbc_gpu(pos: torch.Tensor, r: float, cell: torch.Tensor, max_nu
     saturated = max_num_neighbors > 0 and longest >= int(max_num_neighbors)
     if edges == 0:
         return empty + (saturated,) if return_saturation else empty
-    n0i = n0.to(torch.int64).contiguous()
     if longest <= _row_capacity():
         # rows written in (dst, src, shift) order by the kernel itself
         src = torch.empty(edges, dtype=torch.int64, device=dev)

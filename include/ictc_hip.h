@@ -416,6 +416,22 @@ typedef struct ictc_cell_grid {
     int32_t periodic[3];
 } ictc_cell_grid;
 
+/* Groups atoms by bin, in two calls with an inclusive scan of bin_counts between them:
+ * bins:      for the fractional coordinates [atoms,3] of a cell periodic along all three axes writes the wrap
+ *            image floor(f), f - floor(f) and the bin of each axis; with fractional = NULL (wrap_images
+ *            and wrapped unused) it takes atom_bins as given, each in [0, bins).  Adds each atom to
+ *            bin_counts[1 + bin] ([nbins + 1], zero before) and stores its place in the bin.
+ * bin_atoms: bin_atoms[bin_start[bin] + place] = atom, bin_start = the scanned bin_counts.
+ * The order of a bin's atoms may differ from call to call; the edges of the fills below do not.
+ */
+int ictc_hip_radius_graph_bins(const ictc_cell_grid* grid, const double* fractional, int64_t atoms,
+                               int64_t* wrap_images, double* wrapped, int32_t* atom_bins,
+                               int64_t* bin_counts, int32_t* places, hipStream_t stream);
+
+int ictc_hip_radius_graph_bin_atoms(const ictc_cell_grid* grid, const int32_t* atom_bins, const int32_t* places,
+                                    const int64_t* bin_start, int64_t atoms, int64_t* bin_atoms,
+                                    hipStream_t stream);
+
 int ictc_hip_radius_graph_count(const ictc_cell_grid* grid, const double* wrapped_positions,
                                 const int32_t* atom_bins, const int64_t* bin_start,
                                 const int64_t* bin_atoms, int64_t atoms, int64_t* counts,

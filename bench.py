@@ -411,7 +411,7 @@ def _bench_tp_cfg0(device):
     gbs = BYTES_TP0 * TP0_ROWS / (ms * 1e-3) / 1e9
     traffic = _profile_value("tp_c64_l2_cfg0_kernel_trace_and_traffic.md", "traffic_bytes_per_launch")
     return {"workload": "cfg0 channelwise TP forward C64/lmax2 (11 paths), 65,536 instances, ir_mul",
-            "kernel": "tp_forward_kernel<2,2,2,1>", "mean_launch_ms": ms,
+            "kernel": "tp_forward_kernel<2,2,2,1,false>", "mean_launch_ms": ms,
             "instances_per_s": TP0_ROWS / (ms * 1e-3), "vs_published_11.57M": TP0_ROWS / (ms * 1e-3) / 11.57e6,
             "roofline": {"bound": "hbm", "algorithmic_bytes_per_instance": BYTES_TP0,
                          "algorithmic_bytes_per_launch": BYTES_TP0 * TP0_ROWS, "achieved": gbs,
@@ -468,7 +468,7 @@ def _bench_tp_l4(device):
     and the (4, 4, 3) set on the degree-generic ones (run-time path tables: every set with a degree
     above 3 other than the compiled ones)."""
     out = _tp_degree_leg(device, GEN_L, GEN_L, GEN_L)
-    out["kernels"] = "tp_forward_kernel<4,4,4,1>, tp_backward_wide_kernel<4,4,4>"
+    out["kernels"] = "tp_forward_kernel<4,4,4,1,false>, tp_backward_wide_kernel<4,4,4,false>"
     gen = _tp_degree_leg(device, GEN_L, GEN_L, GEN_L - 1)
     gen["kernels"] = "gen_tp_forward_kernel, gen_tp_backward_kernel"
     out["generic_443"] = gen
@@ -850,8 +850,8 @@ def _bench_linear(device):
                 "algorithmic_bytes": nbytes, "hbm_frac": nbytes / (ms * 1e-3) / 1e9 / HBM_PEAK_GBS}
     return {"workload": "cfg4 MACE message linear (interaction 2): per-degree path blocks 4/6/7/6 x C128 -> C128, "
                         "2,048 atoms, fp32",
-            "forward": leg(fwd_ms, dense[0], "degree_linear_kernel<0, true, 2, 64>"),
-            "input_grad": leg(grad_ms, dense[1], "degree_linear_kernel<1, true, 1, 128>"),
+            "forward": leg(fwd_ms, dense[0], "degree_linear_split_kernel<0, 128>"),
+            "input_grad": leg(grad_ms, dense[1], "degree_linear_input_grad_kernel<8>"),
             "weight_grad": leg(wgrad_ms, dense[2], "degree_linear_wgrad_kernel<0> + degree_linear_wgrad_sum_kernel")}
 
 

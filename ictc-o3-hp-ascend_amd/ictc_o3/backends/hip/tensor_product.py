@@ -227,6 +227,11 @@ def packed_tensor_product(plan: TensorProductPlan, features: torch.Tensor, harmo
     """Packed ir_mul TP: features [E, C(L_in+1)^2], harmonics [E,(L_e+1)^2],
     gates [E, P*C] -> [E, NOC*C].  The path weights are folded into the gates already, or passed as
     ``weight`` [P*C] for the kernels to fold (see ``gates_and_weight``)."""
+    if weight is not None and (not plan.is_full or weight.shape != (plan.full_gate_width,)
+                               or weight.dtype != torch.float32 or weight.device != gates.device
+                               or not weight.is_contiguous()):
+        raise ValueError("A path weight for the kernels must be contiguous float32 [P*C] on the gates' device, "
+                         "for a plan of every path")
     if plan.is_full:
         return _Forward.apply(plan, features.contiguous(), harmonics.contiguous(), gates.contiguous(), weight)
     rows, c = gates.shape[0], plan.channels
@@ -242,12 +247,14 @@ def packed_tensor_product(plan: TensorProductPlan, features: torch.Tensor, harmo
 def gates_and_weight(owner, plan: TensorProductPlan, gates: Optional[torch.Tensor], rows: int):
     """(gates [E, P*C], path weight [P*C] or None) for ``packed_tensor_product``: the owner's
     per-(path, channel) weight is left to the kernels when nothing differentiates it and they take it
-    (every path of a compiled degree set, P*C up to ``weight_capacity``), which saves a pass over the
-    gates and one over their gradients; otherwise it is multiplied into the gates here
+    (every path of a compiled degree set, P*C up to ``weight_capacity``; they read P*C floats, so a weight
+    that broadcasts against [P, C] does not go there), which saves a pass over the gates and one
+    over their gradients; otherwise it is multiplied into the gates here
     (``owner.effective_gates``).  Both read the weight on every call and round the same products."""
     w = owner.weight
     if (gates is None or not plan.is_full or plan.full_gate_width > plan.weight_capacity
-            or w.device != gates.device or (w.requires_grad and torch.is_grad_enabled())):
+            or w.shape != (plan.num_paths, plan.channels) or w.device != gates.device
+            or (w.requires_grad and torch.is_grad_enabled())):
         return owner.effective_gates(gates, rows), None
     return gates.reshape(rows, plan.full_gate_width), w.detach().reshape(-1).contiguous()
 

@@ -1,0 +1,43 @@
+"""What the tensor product's path weight must be for the kernels to fold it into the gates
+(``gates_and_weight``): every other weight takes the separate product ``gates * weight``, as before the
+kernels took one.  CPU only (no kernel runs)."""
+import pytest
+import torch
+
+from ictc_o3.backends.hip import tensor_product as T
+from ictc_o3.basis.ictd_irreps import EdgeWeightedPathPreservingTensorProduct
+
+ROWS, C = 3, 4
+
+
+def _owner(lmax=2):
+    owner = EdgeWeightedPathPreservingTensorProduct(C, lmax, internal_compute_dtype=torch.float32)
+    owner.weight.requires_grad_(False)
+    plan = owner.hip_plan(lmax, lmax)
+    assert plan.is_full and plan.weight_capacity >= owner.num_paths * C
+    return owner, plan, torch.randn(ROWS, owner.num_paths * C)
+
+
+@pytest.mark.parametrize("shape", [(1, C), (None, 1), (1, 1), (C,), (1, None, C)])
+def test_broadcast_weights_take_the_separate_product(shape):
+    """The kernels read P * C floats: a weight that broadcasts against [P, C] holds fewer."""
+    owner, plan, gates = _owner()
+    shape = tuple(owner.num_paths if n is None else n for n in shape)
+    owner.weight = torch.nn.Parameter(torch.randn(shape), requires_grad=False)
+    product, weight = T.gates_and_weight(owner, plan, gates, ROWS)
+    assert weight is None
+    want = gates.reshape(ROWS, owner.num_paths, C) * owner.weight
+    assert torch.equal(product, want.reshape(ROWS, -1))
+
+
+def test_a_passed_weight_is_checked():
+    owner, plan, gates = _owner()
+    x, y = torch.randn(ROWS, 9 * C), torch.randn(ROWS, 9)
+    n = owner.num_paths * C
+    for bad in (torch.ones(n - 1), torch.ones(owner.num_paths, C), torch.ones(n, dtype=torch.float64),
+                torch.ones(2 * n)[::2], torch.ones(n, device="meta")):
+        with pytest.raises(ValueError):
+            T.packed_tensor_product(plan, x, y, gates, bad)
+    some = T.TensorProductPlan(owner.paths[1:], C, 2, 2, 2)        # a path subset does not take one
+    with pytest.raises(ValueError):
+        T.packed_tensor_product(some, x, y, gates[:, C:], torch.ones(n - C))

@@ -144,11 +144,14 @@ def _add(acc, value):
 
 class _Forward(torch.autograd.Function):
     """w: a frozen path weight folded into the gates, or None (a constant of the map: the map and
-    every derivative of it stay trilinear in x, Y and g)."""
+    every derivative of it stay trilinear in x, Y and g).  A recorded call keeps a copy of w (at most
+    16 KB): the owner may change its weight before the backward, also through ``weight.data``."""
 
     @staticmethod
     def forward(ctx, plan, x, y, g, w=None):
         ctx.plan = plan
+        if w is not None and any(ctx.needs_input_grad[1:4]):
+            w = w.clone()
         ctx.save_for_backward(x, y, g, w)
         return _forward_raw(plan, x, y, g, w)
 

@@ -41,3 +41,31 @@ def test_a_passed_weight_is_checked():
     some = T.TensorProductPlan(owner.paths[1:], C, 2, 2, 2)        # a path subset does not take one
     with pytest.raises(ValueError):
         T.packed_tensor_product(some, x, y, gates[:, C:], torch.ones(n - C))
+
+
+@pytest.mark.parametrize("change", [lambda w: w.data.mul_(3.0), lambda w: w.mul_(3.0)], ids=["data", "in place"])
+def test_the_backward_uses_the_weight_of_its_forward(monkeypatch, change):
+    """A weight that changes between a forward and its backward, where only the features are
+    differentiated: the gradient is that of the product that was computed."""
+    owner, plan, gates = _owner()
+    seen = []
+
+    def kernels(plan, x, y, g, w=None):
+        seen.append(w)
+        return x.new_zeros(ROWS, plan.full_out_width)
+
+    def adjoint(plan, need, x, y, g, go, w=None):
+        seen.append(w.clone())
+        return torch.zeros_like(x), None, None
+
+    monkeypatch.setattr(T, "_forward_raw", kernels)
+    monkeypatch.setattr(T, "_backward_raw", adjoint)
+    x, y = torch.randn(ROWS, 9 * C), torch.randn(ROWS, 9)
+    before = owner.weight.reshape(-1).clone()
+    out = T.packed_tensor_product(plan, x.requires_grad_(), y, *T.gates_and_weight(owner, plan, gates, ROWS))
+    change(owner.weight)
+    out.sum().backward()
+    assert len(seen) == 2 and torch.equal(seen[1], before)
+    # nothing to differentiate: no copy
+    T.packed_tensor_product(plan, x.detach(), y, *T.gates_and_weight(owner, plan, gates, ROWS))
+    assert seen[2].data_ptr() == owner.weight.data_ptr()

@@ -232,9 +232,9 @@ def packed_tensor_product(plan: TensorProductPlan, features: torch.Tensor, harmo
     ``weight`` [P*C] for the kernels to fold (see ``gates_and_weight``)."""
     if weight is not None and (not plan.is_full or weight.shape != (plan.full_gate_width,)
                                or weight.dtype != torch.float32 or weight.device != gates.device
-                               or not weight.is_contiguous()):
-        raise ValueError("A path weight for the kernels must be contiguous float32 [P*C] on the gates' device, "
-                         "for a plan of every path")
+                               or not weight.is_contiguous() or (weight.requires_grad and torch.is_grad_enabled())):
+        raise ValueError("A path weight for the kernels must be frozen, contiguous float32 [P*C] on the gates' "
+                         "device, for a plan of every path")
     if plan.is_full:
         return _Forward.apply(plan, features.contiguous(), harmonics.contiguous(), gates.contiguous(), weight)
     rows, c = gates.shape[0], plan.channels
@@ -259,7 +259,7 @@ def gates_and_weight(owner, plan: TensorProductPlan, gates: Optional[torch.Tenso
             or w.shape != (plan.num_paths, plan.channels) or w.device != gates.device
             or (w.requires_grad and torch.is_grad_enabled())):
         return owner.effective_gates(gates, rows), None
-    return gates.reshape(rows, plan.full_gate_width), w.detach().reshape(-1).contiguous()
+    return gates.reshape(rows, plan.full_gate_width), w.reshape(-1).contiguous()
 
 
 def blocks_to_packed(blocks: Dict[int, torch.Tensor], lmax: int) -> torch.Tensor:

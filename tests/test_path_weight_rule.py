@@ -35,7 +35,7 @@ def test_a_passed_weight_is_checked():
     x, y = torch.randn(ROWS, 9 * C), torch.randn(ROWS, 9)
     n = owner.num_paths * C
     for bad in (torch.ones(n - 1), torch.ones(owner.num_paths, C), torch.ones(n, dtype=torch.float64),
-                torch.ones(2 * n)[::2], torch.ones(n, device="meta")):
+                torch.ones(2 * n)[::2], torch.ones(n, device="meta"), torch.ones(n, requires_grad=True)):
         with pytest.raises(ValueError):
             T.packed_tensor_product(plan, x, y, gates, bad)
     some = T.TensorProductPlan(owner.paths[1:], C, 2, 2, 2)        # a path subset does not take one
@@ -69,3 +69,19 @@ def test_the_backward_uses_the_weight_of_its_forward(monkeypatch, change):
     # nothing to differentiate: no copy
     T.packed_tensor_product(plan, x.detach(), y, *T.gates_and_weight(owner, plan, gates, ROWS))
     assert seen[2].data_ptr() == owner.weight.data_ptr()
+
+
+def test_a_forward_mode_tangent_is_not_dropped(monkeypatch):
+    """The product has no forward-mode derivative: a weight with a tangent has to reach it with its
+    tangent, so that the call is refused and not answered as if there were none."""
+    import torch.autograd.forward_ad as fwad
+    owner, plan, gates = _owner()
+    monkeypatch.setattr(T, "_forward_raw", lambda plan, x, y, g, w=None: x.new_zeros(ROWS, plan.full_out_width))
+    with fwad.dual_level():
+        del owner.weight
+        owner.weight = fwad.make_dual(torch.ones(owner.num_paths, C), torch.ones(owner.num_paths, C))
+        weight = T.gates_and_weight(owner, plan, gates, ROWS)[1]
+        assert fwad.unpack_dual(weight).tangent is not None
+        x, y = torch.randn(ROWS, 9 * C), torch.randn(ROWS, 9)
+        with pytest.raises(RuntimeError, match="jvp"):
+            T.packed_tensor_product(plan, x, y, gates, weight)

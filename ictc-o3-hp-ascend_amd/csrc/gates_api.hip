@@ -160,17 +160,19 @@ gates_forward_kernel(const float* __restrict__ h, const float* __restrict__ w, i
         const uint32_t voff = 4u * half * ld + n * 4u;
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
-          const f32x2 v{acc[t][0][i], acc[t][1][i]};
+          const f32x2 v{acc[t][0][i] * kSplitUnscale, acc[t][1][i] * kSplitUnscale};
           __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v), ro, voff,
                                                 (32 * t + mfma_row(i, 0)) * ld, kNonTemporal);
         }
       } else {
+        uint32_t step = ld;                  // opaque: the 32 row offsets are formed here, not kept through the loop
+        asm volatile("" : "+s"(step));
 #pragma unroll
         for (int i = 0; i < 16; ++i)
 #pragma unroll
           for (int ct = 0; ct < 2; ++ct)
-            buf_store<1>(ro, n + ct < N ? (32 * t + mfma_row(i, half)) * ld + (n + ct) * 4u : 0xFFFFFFF0u,
-                         Vec<1>{{acc[t][ct][i]}});
+            buf_store<1>(ro, n + ct < N ? (32 * t + mfma_row(i, half)) * step + (n + ct) * 4u : 0xFFFFFFF0u,
+                         Vec<1>{{acc[t][ct][i] * kSplitUnscale}});
       }
     }
     if (more) wr.store(tile[(ch + 1) & 1]);
@@ -277,7 +279,7 @@ gates_input_grad_kernel(const float* __restrict__ g, int64_t ldg, const float* _
 #pragma unroll
   for (int ct = 0; ct < 2; ++ct)
 #pragma unroll
-    for (int i = 0; i < 16; ++i) hi[0][ct][i] += lo[0][ct][i];
+    for (int i = 0; i < 16; ++i) hi[0][ct][i] = (hi[0][ct][i] + lo[0][ct][i]) * kSplitUnscale;
 #pragma unroll
   for (int ct = 0; ct < 2; ++ct) {
     const int c = 32 * ct + r;
@@ -391,7 +393,7 @@ gates_weight_grad_kernel(const float* __restrict__ g, int64_t ldg, const float* 
     split_g(1, next);
     step(tile[b], 0);
 #pragma unroll
-    for (int q = 0; q < 24; ++q) {
+    for (int q = 0; q < 4 * kSplitProducts; ++q) {
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);   // one matrix instruction
       __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);   // four VALU instructions
     }
@@ -401,7 +403,7 @@ gates_weight_grad_kernel(const float* __restrict__ g, int64_t ldg, const float* 
     split_g(0, next);
     step(tile[b], 1);
 #pragma unroll
-    for (int q = 0; q < 24; ++q) {
+    for (int q = 0; q < 4 * kSplitProducts; ++q) {
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
       __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);
     }
@@ -414,6 +416,7 @@ gates_weight_grad_kernel(const float* __restrict__ g, int64_t ldg, const float* 
   for (int t = 0; t < 2; ++t)
 #pragma unroll
     for (int ct = 0; ct < 2; ++ct) {
+      unscale(acc[t][ct]);
       const bool redo = any_nonfinite(acc[t][ct]);
 #pragma unroll
       for (int i = 0; i < 16; ++i) {

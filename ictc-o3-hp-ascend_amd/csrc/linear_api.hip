@@ -420,7 +420,7 @@ degree_linear_split_kernel(const float* __restrict__ in, float* __restrict__ out
           ++n;
         }
         if (rho0 + v >= g.rows || col >= ncols) continue;
-        float val = hi[0][t][4 * q + v];
+        float val = hi[0][t][4 * q + v] * kSplitUnscale;
         if (redo) {
           val = 0.f;
           for (int k = 0; k < kdim; ++k) {
@@ -538,7 +538,7 @@ degree_linear_input_grad_kernel(const float* __restrict__ gy, float* __restrict_
     const bool redo = any_nonfinite(acc[0][0]) || any_nonfinite(acc[0][1]);   // see split_bf16.hpp: again in fp32
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
-      f32x2 v{acc[0][0][i], acc[0][1][i]};
+      f32x2 v{acc[0][0][i] * kSplitUnscale, acc[0][1][i] * kSplitUnscale};
       if (redo) {
         v = f32x2{0.f, 0.f};
         const int64_t rho = row0 + mfma_row(i, half);
@@ -832,7 +832,7 @@ degree_linear_wgrad_kernel(const float* __restrict__ gy, const float* __restrict
   for (int i = 0; i < 16; ++i) {
     const int o = o0 + o_t + mfma_row(i, half);
     if (o >= O || j >= g.k) continue;
-    float v = acc[0][0][i];
+    float v = acc[0][0][i] * kSplitUnscale;
     if (redo) {
       v = 0.f;
       for (int64_t rho = r0; rho < r1; ++rho) {

@@ -776,13 +776,14 @@ int launch_msg_forward_tangent(const ictc_tp_desc& d, const float* x, const floa
 // One block per (receiver, 64-channel chunk), of msg_grad_waves waves; path k's U block is built by wave
 // k mod 4 (mod 8 in the larger blocks), then each wave walks its share of the receiver's edges.
 // Bound by HBM: the gates in, their gradient and dxe out (3.3 GB for C = 128, lmax 3, 106,304 edges: 680 us at
-// a large copy's 4.9 TB/s).  No wait in the edge loop may take in more than it needs: indices and
-// harmonics come by vector loads (scalar loads share their counter with the LDS reads), the next
-// edge's loads are in flight throughout, and the next U row's reads behind the current row's products, with
-// no branch in between (WY, ACC are template parameters).  At that size the four launches take
-// 0.95 ms, without the harmonics gradient 0.75 ms, the tangent without it 1.03 ms (before: scalar index and harmonics
-// loads in the loop, 4 waves per block: 1.05, 0.83 and 1.10 ms); 5,219 edges over 256 receivers, C = 64,
-// lmax 2: 26 us (49 us); outputs bit-identical.  dY partials [edges, chunks, NY]: group launches run
+// a large copy's 4.9 TB/s).  The next edge's loads are in flight throughout, the harmonics by vector loads
+// (a scalar load in flight shares its counter with the LDS reads: 2.4 ms instead of 1.24 for the tangent with the
+// harmonics gradient, lmax 3), the next U row's reads behind the current row's products, with no branch in
+// between (WY, ACC are template parameters).  The edge's index and source stay scalar loads: 64 of them
+// loaded at once, one per lane, and read back by v_readlane cost 15 % of a lmax-1 launch and 2 to 8 % above.
+// C = 128, lmax 3, 107,756 edges, four launches: 0.92 ms, without the harmonics gradient 0.77, the tangent
+// without it 1.03 ms (before the pipeline, with 4 waves per block: 1.06, 0.87 and 1.10 ms).  Outputs are
+// bit-identical for every block size.  dY partials [edges, chunks, NY]: group launches run
 // in order on one stream; the first writes each (edge, chunk) slot, later groups add to it (a fixed
 // order; the caller sums the chunk axis).
 struct NodeU {
@@ -810,50 +811,26 @@ struct NodeUOf {
 // The compiler forms v before this point.
 __device__ __forceinline__ void pin(float& v) { asm volatile("" : "+v"(v)); }
 
-// The edges of one wave of a receiver's block: wave w takes the slots s0 + w, s0 + w + waves, ... of the
-// receiver's CSR range.  The indices and sources of 64 of them are loaded at once, one per lane, and
-// read back lane by lane, so that an edge has no chain of index loads (perm -> src -> rows) in front of
-// its own loads and no scalar load in flight beside its LDS reads (both share one counter, and scalar
-// loads return out of order, so a wait for either is a wait for all).
-struct WaveEdges {
-  const int64_t *perm, *src;
-  int64_t s1, slot;   // end of the range; next slot
-  int waves, lane, at;
-  uint32_t elo, ehi, sl;
-  __device__ __forceinline__ WaveEdges(const int64_t* perm_, const int64_t* src_, int64_t s0, int64_t s1_, int wave,
-                                       int waves_, int lane_)
-      : perm(perm_), src(src_), s1(s1_), slot(s0 + wave), waves(waves_), lane(lane_), at(kWave - 1), elo(0), ehi(0),
-        sl(0) {}
-  __device__ __forceinline__ bool more() const { return slot < s1; }
-  __device__ __forceinline__ int64_t next() {   // more() only
-    at = (at + 1) & (kWave - 1);
-    if (at == 0) {   // wave-uniform
-      int64_t s = slot + static_cast<int64_t>(lane) * waves;
-      s = s < s1 ? s : s1 - 1;
-      const int64_t e = perm ? perm[s] : s;
-      elo = static_cast<uint32_t>(e);
-      ehi = static_cast<uint32_t>(static_cast<uint64_t>(e) >> 32);
-      sl = static_cast<uint32_t>(src[e]);
-    }
-    slot += waves;
-    const uint32_t lo = __builtin_amdgcn_readlane(elo, at), hi = __builtin_amdgcn_readlane(ehi, at);
-    return static_cast<int64_t>(static_cast<uint64_t>(hi) << 32 | lo);
-  }
-  __device__ __forceinline__ uint32_t source() const { return __builtin_amdgcn_readlane(sl, at); }   // of next()'s
-};
-
 constexpr int kMsgGradWaves = 16;   // most waves of a block (128 VGPRs)
 
-// Waves per block, each walking its share of the receiver's edges beside one U table.  A block's LDS (50 KB
-// for input degree 3 at lmax 3) allows three blocks per CU, so 4 waves per block leave 3 waves per SIMD
-// to hide an edge's loads; 8 give 4 to 5.  Measured with 4, 8 and 16 waves (us; first order with
-// harmonics gradient / tangent without): C = 128, lmax 3, 106,304 edges over 2,048 receivers 1020 / 1084,
-// 987 / 1044, 1067 / 1096; C = 64, lmax 2, 852,297 edges over 16,384 receivers 1514 / 1876, 1618 / 1840, 1976 /
-// 1964 (with the harmonics gradient the channel sums' exchanges bound the denser waves); a launch of
-// at most two blocks per CU, C = 64, lmax 2, 5,219 edges over 256 receivers 49 / 46, 33 / 31, 26 / 26.
+// Waves per block, each walking its share of the receiver's edges beside one U table.  16 where the
+// launch leaves the chip idle (at most two blocks per CU): a receiver's 52 edges then take four rounds.
+// Otherwise 8: a block's LDS (50 KB for input degree 3 at lmax 3) allows three blocks per CU, so 4 waves
+// would leave 3 per SIMD to hide an edge's loads.  4 for long launches with the harmonics gradient below
+// input degree 3, whose channel sums' exchanges bound the denser waves.  us with 4, 8 and 16 waves, first
+// order with harmonics gradient / tangent without, 52 edges per receiver, C = 64, by blocks:
+//            lmax 1                                lmax 2                                lmax 3
+//    256     35 23 17 / 34 22 18                   86 54 41 / 74 48 44                   163 98 79 / 153 99 93
+//    600     45 36 34 / 42 38 36                   109 84 89 / 99 100 93                 202 181 174 / 220 213 201
+//   1200     58 58 56 / 65 65 62                   143 143 154 / 171 169 161             337 303 305 / 395 366 352
+//   2400     108 98 98 / 125 116 112               269 252 287 / 317 299 301             602 548 588 / 676 635 644
+//   4800     185 179 184 / 226 216 212             476 472 560 / 586 566 577
+//   9600     345 345 363 / 432 414 411             899 909 1102 / 1142 1106 1128
+//  16384     569 573 614 / 723 697 697             1489 1531 1865 / 1922 1865 1914
 inline int msg_grad_waves(int lin, bool harmonics, int64_t blocks) {
-  if (blocks <= 2 * static_cast<int64_t>(compute_units())) return kMsgGradWaves;
-  return lin >= 3 || !harmonics ? 8 : 4;
+  const int64_t cus = compute_units();
+  if (blocks <= 2 * cus) return kMsgGradWaves;
+  return lin >= 3 || !harmonics || blocks <= 32 * cus ? 8 : 4;
 }
 
 template <int LIN, int LE, int LOUT, int L1, bool JVP, bool ACC, bool WY>
@@ -925,8 +902,7 @@ msg_edge_grad_degree_kernel(const float* __restrict__ x, const float* __restrict
   const int wjc = wj < NY ? wj : NY - 1;
   const int yj = lane < NY ? lane : NY - 1;
   // One edge's inputs: its harmonics rows (one value per lane), the source features of degree l1, the
-  // group's gates and the harmonics partial that earlier degree launches left in the slot.  All vector
-  // loads: a scalar load in flight would make the first LDS wait below wait for it too.
+  // group's gates and the harmonics partial that earlier degree launches left in the slot, by vector loads.
   struct EdgeIn {
     float yl[NT];
     float xr[NT][NI];
@@ -1051,21 +1027,23 @@ msg_edge_grad_degree_kernel(const float* __restrict__ x, const float* __restrict
       if (wown) dyp[(e * nchunks + chunk) * NY + wj] = in.prev + tot;
     }
   };
-  // Software pipeline over the wave's edges: an edge's loads are issued before the edge ahead of it is
-  // computed and stored.
-  WaveEdges list(perm, src, rowptr[node], rowptr[node + 1], wave, waves, lane);
-  if (list.more()) {
+  // Software pipeline over the wave's edges (slots wave, wave + waves, ... of the receiver's range): an
+  // edge's loads are issued before the edge ahead of it is computed and stored.
+  const int64_t s1 = rowptr[node + 1];
+  int64_t slot = rowptr[node] + wave;
+  if (slot < s1) {
     EdgeIn cur;
-    int64_t e = list.next();
-    fetch(e, list.source(), cur);
+    int64_t e = perm ? perm[slot] : slot;
+    fetch(e, static_cast<uint32_t>(src[e]), cur);
 #pragma clang loop unroll(disable)
     for (;;) {
-      const bool more = list.more();
+      slot += waves;
+      const bool more = slot < s1;
       int64_t ne = e;
       EdgeIn nxt;
       if (more) {
-        ne = list.next();
-        fetch(ne, list.source(), nxt);
+        ne = perm ? perm[slot] : slot;
+        fetch(ne, static_cast<uint32_t>(src[ne]), nxt);
       }
       compute(e, cur);
       if (!more) break;

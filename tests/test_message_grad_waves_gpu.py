@@ -1,6 +1,6 @@
 """Edge gradients of the message kernels at every block size of their dispatch (4, 8 and 16 waves):
-receivers with no edge, with fewer edges than the block has waves, and with more than the 64 edges per wave
-whose indices a wave loads at once, against the oracle's autograd in float64."""
+receivers with no edge, with fewer edges than the block has waves, and with many rounds of edges for each
+wave and one more for some, against the oracle's autograd in float64."""
 import pytest
 import torch
 
@@ -11,13 +11,14 @@ from test_message_gpu import _edge_inputs, _op
 pytestmark = pytest.mark.gpu
 
 
-# more than two blocks per CU (513 receivers of one chunk on 256 CUs) or fewer, and the waves there
+# up to two blocks per CU (512 receivers of one chunk on 256 CUs), up to 32 and above, and the waves there
 @pytest.mark.parametrize("lmax,receivers,harmonics,waves", [
-    (2, 530, True, 4), (2, 530, False, 8), (3, 530, True, 8), (3, 530, False, 8), (2, 20, True, 16), (3, 20, True, 16),
+    (2, 8200, True, 4), (1, 8200, True, 4), (2, 8200, False, 8), (2, 530, True, 8), (2, 530, False, 8),
+    (3, 530, True, 8), (3, 530, False, 8), (2, 20, True, 16), (3, 20, True, 16),
     (3, 20, False, 16)])
 def test_edge_gradients(gpu, lmax, receivers, harmonics, waves):
     c = 40                                           # a ragged chunk: lanes past the channels
-    many = 64 * waves + waves // 2 + 1               # a second round of indices in some waves only
+    many = 64 * waves + waves // 2 + 1               # a last round of edges in some waves only
     counts = torch.arange(receivers) % 3             # 0, 1, 2 edges
     counts[1] = many
     counts[-1] = waves + 1

@@ -4,15 +4,20 @@ three bf16 parts on the matrix cores): the radial network's last layer ``h W^T``
 weight adjoint ``g^T h``.  ``product`` recognises the three forms in ``a @ b``; ``linear.mm`` asks
 it first and keeps its library routes for every other shape.
 
-The lines between the routes (MI355X, us per call with its launches, the library's time in brackets):
+The lines between the routes (MI355X, us per call in a replayed graph, the library's time in brackets):
 
-* forward from 2,048 rows: 10 (13) at 2,048 x 2,944, 25 (34) at 8,192 x 2,944, 275 (385) at 105,634 x
-  2,944, 38 (57) at 105,634 x 352; below, both are the launch;
+* forward from 2,048 rows and 3.5 M results: a block has its rows to load and split before its first
+  product, so that a small launch takes 6 us whatever its size: 6.0 (2.7) at 2,048 x 128, 6.9 (5.8) at 5,500 x
+  352, 7.0 (6.2) at 3,500 x 704, 6.9 (5.7) at 20,000 x 128; from the line on 7.6 (8.6) at 7,000 x 512, 10.0 (12.3)
+  at 2,048 x 2,944, 11.5 (14.7) at 20,000 x 352, 288 (408) at 105,634 x 2,944, and at worst 9.8 (9.2) at 20,000 x 256;
 * input adjoint from 50,000 rows: a block takes 128 rows and a fixed 1.1 us per 32 columns, so fewer
-  rows leave CUs idle: 116 (106) at 32,768 x 2,944, 169 (220) at 50,000 x 2,944, 300 (353) at 105,634 x
-  2,944, 48 (54) at 50,000 x 704;
-* weight adjoint from 2,048 rows: 24 (68) at 2,048 x 2,944, 18 (28) at 8,192 x 352, 287 (620) at 105,634 x
-  2,944; up to 4,096 rows and 704 columns the two are within 3 us of each other.
+  rows leave CUs idle: 105 (88) at 8,192 x 2,944, 120 (108) at 32,768 x 2,944, 176 (225) at 50,000 x 2,944, 40 (40) at
+  65,000 x 512, 81 (94) at 105,634 x 704, 311 (373) at 105,634 x 2,944.  A second round of blocks begins above
+  131,072 rows and costs 36 us at 2,944 columns, less than the lead: 365 (466) at 131,072, 401 (480) at 131,200,
+  418 (481) at 140,000, 599 (714) at 211,000; 59 (60) at 131,200 x 352, 28 (28) at 140,000 x 128;
+* weight adjoint from 4,096 rows, or 2,048 from 640 columns: 15 (11) at 2,048 x 128, 15 (12) at 2,048 x 512, 17 (16)
+  at 4,000 x 512; 16 (18) at 2,048 x 704, 17 (33) at 8,000 x 128, 22 (23) at 8,000 x 704, 19 (25) at 16,000 x 128,
+  156 (216) at 105,634 x 1,408.
 """
 from __future__ import annotations
 
@@ -25,8 +30,11 @@ from ... import _lib
 WIDTH = 64
 MIN_OUTER = 128            # narrower outer sides stay on the library (its 64 x 64 products take one tile)
 FORWARD_ROWS = 2048
+FORWARD_RESULTS = 3_500_000
 INPUT_GRAD_ROWS = 50000
 WEIGHT_GRAD_ROWS = 2048
+WEIGHT_GRAD_NARROW = 640   # narrower outer sides ...
+WEIGHT_GRAD_NARROW_ROWS = 4096   # ... from these rows
 MAX_OUTER = 1 << 20
 MAX_ROW_STRIDE = 1 << 22
 
@@ -86,22 +94,26 @@ def product(a: torch.Tensor, b: torch.Tensor, out: Optional[torch.Tensor] = None
     """a [M, K] @ b [K, N] when it is one of the three forms at a size they are the faster route
     for; None otherwise.  out: a caller's row-major result (the first two forms; a row slice of a
     wider matrix for the first)."""
-    if not a.is_cuda or a.dtype != torch.float32 or b.dtype != torch.float32 or a.device != b.device:
-        return None
     m, k = a.shape
     n = b.shape[1]
-    if k == WIDTH:
-        if (FORWARD_ROWS <= m and MIN_OUTER <= n <= MAX_OUTER and _hidden(a) and _weight(b.t())
-                and (out is None or _rows(out, n))):
-            return _forward(a, b.t(), out)
+    outer = m if n == WIDTH else n
+    # sizes first: a small call's products end here
+    forward = k == WIDTH and m >= FORWARD_ROWS and m * n >= FORWARD_RESULTS and MIN_OUTER <= n <= MAX_OUTER
+    input_grad = n == WIDTH and m >= INPUT_GRAD_ROWS and MIN_OUTER <= k <= MAX_OUTER and k % 4 == 0
+    weight_grad = (k >= WEIGHT_GRAD_ROWS and (n == WIDTH or m == WIDTH) and out is None
+                   and MIN_OUTER <= outer <= MAX_OUTER
+                   and (k >= WEIGHT_GRAD_NARROW_ROWS or outer >= WEIGHT_GRAD_NARROW))
+    if not (forward or input_grad or weight_grad) or not a.is_cuda or a.device != b.device:
         return None
-    if (n == WIDTH and m >= INPUT_GRAD_ROWS and MIN_OUTER <= k <= MAX_OUTER and k % 4 == 0 and _rows(a, k)
-            and a.stride(0) % 4 == 0 and a.data_ptr() % 16 == 0 and _weight(b)
+    if a.dtype != torch.float32 or b.dtype != torch.float32:
+        return None
+    if forward and _hidden(a) and _weight(b.t()) and (out is None or _rows(out, n)):
+        return _forward(a, b.t(), out)
+    if (input_grad and _rows(a, k) and a.stride(0) % 4 == 0 and a.data_ptr() % 16 == 0 and _weight(b)
             and (out is None or (out.stride(0) == WIDTH and out.stride(1) == 1))):
         return _input_grad(a, b, out)
-    if k >= WEIGHT_GRAD_ROWS and out is None:
-        if n == WIDTH and MIN_OUTER <= m <= MAX_OUTER and _rows(a.t(), m) and b.stride(1) == 1 and b.stride(0) == WIDTH:
-            return _weight_grad(a.t(), b, False)
-        if m == WIDTH and MIN_OUTER <= n <= MAX_OUTER and _rows(b, n) and a.stride(0) == 1 and a.stride(1) == WIDTH:
-            return _weight_grad(b, a.t(), True)
+    if weight_grad and n == WIDTH and _rows(a.t(), m) and b.stride(1) == 1 and b.stride(0) == WIDTH:
+        return _weight_grad(a.t(), b, False)
+    if weight_grad and m == WIDTH and _rows(b, n) and a.stride(0) == 1 and a.stride(1) == WIDTH:
+        return _weight_grad(b, a.t(), True)
     return None

@@ -81,7 +81,7 @@ def test_non_finite_and_huge_values_as_in_float32():
 
 
 def test_rule_takes_the_three_forms_and_leaves_the_rest(monkeypatch):
-    for name in ("FORWARD_ROWS", "INPUT_GRAD_ROWS", "WEIGHT_GRAD_ROWS"):
+    for name in ("FORWARD_ROWS", "FORWARD_RESULTS", "INPUT_GRAD_ROWS", "WEIGHT_GRAD_ROWS", "WEIGHT_GRAD_NARROW_ROWS"):
         monkeypatch.setattr(G, name, 256)
     h, w, g = _inputs(300, 132)
     for a, b in ((h, w.t()), (h, w.t().contiguous()), (g, w), (g, w.t().contiguous().t()), (g.t(), h), (h.t(), g)):
@@ -95,3 +95,15 @@ def test_rule_takes_the_three_forms_and_leaves_the_rest(monkeypatch):
         assert G.product(a, b) is None
     for a, b in refused[:-1]:
         assert torch.allclose(L._product(a, b), (a.double() @ b.double()).float(), rtol=1e-4, atol=1e-4)
+
+
+@pytest.mark.parametrize("rows,width,forward,weight", [
+    (6835, 512, False, True), (6836, 512, True, True), (2048, 1708, False, True), (2048, 1709, True, True),
+    (2047, 2944, False, False), (27000, 128, False, True), (4095, 636, False, False), (4095, 640, False, True),
+    (4096, 128, False, True)])
+def test_lines_of_the_rule(rows, width, forward, weight):
+    h, w, g = _inputs(rows, width)
+    for a, b, taken in ((h, w.t(), forward), (g.t(), h, weight), (h.t(), g, weight), (g, w, False)):
+        got = G.product(a, b)
+        assert (got is not None) is taken
+        _close(L._product(a, b), a, b)

@@ -758,7 +758,8 @@ def _bench_mace(device):
     return {"workload": "cfg4 MACE C128/lmax3, 2 interactions, correlation 3, 2,048 atoms, r_c 5 A",
             "edges": graph["edge_src"].numel(),
             "step_roofline": {"what": "sum of the modelled work at its own roofline (unique bytes at 8 TB/s, "
-                                      "useful FLOPs at 157.3 TFLOP/s) over the HIP-graph replay time",
+                                      "useful FLOPs at 157.3 TFLOP/s, split-bf16 products at 417) over the HIP-graph "
+                                      "replay time",
                               **floor},
             "inference": leg(infer_ms, 11.0e3, "eager"),
             "training": leg(train_ms, 3.81e3, "eager"),
@@ -805,14 +806,16 @@ def _bench_mace_steps(device, modes=("inference", "training"), replays: int = 20
     return out
 
 
-LIN_COUNTS, LIN_C, MFMA_F32_PEAK_TFLOPS = (4, 6, 7, 6), 128, 157.3   # fp32 MFMA, dense (published)
+LIN_COUNTS, LIN_C = (4, 6, 7, 6), 128
+MFMA_F32_PEAK_TFLOPS = 157.3                    # fp32 MFMA, dense (published)
+MFMA_SPLIT_PEAK_TFLOPS = 2500.0 / 6             # fp32 product as six bf16 part products (bf16 MFMA, dense, published)
 
 
 def _bench_linear(device):
     """The second interaction's message linear of the cfg-4 MACE step (per degree 4 / 6 / 7 / 6
     path blocks of C = 128 channels into 128, 2,048 atoms, alpha = 1/avg_num_neighbors) on the
-    fp32-MFMA kernels, forward, input adjoint and weight adjoint, beside the dense-GEMM routes
-    they replaced (per-degree rearranged copies, rocBLAS products, concatenation)."""
+    split-bf16 MFMA kernels, forward, input adjoint and weight adjoint, beside the dense-GEMM
+    routes they replaced (per-degree rearranged copies, library products, concatenation)."""
     from ictc_o3.backends.hip.degree_linear import DegreeLinearPlan, _forward_raw, _input_grad_raw, _weight_grad_raw
     from ictc_o3.backends.hip.linear import mm
     n, c, alpha = MACE_ATOMS, LIN_C, 1.0 / 50.0
@@ -845,8 +848,8 @@ def _bench_linear(device):
     def leg(ms, dense_ms, kernel):
         tf = flops / (ms * 1e-3) / 1e12
         return {"kernel": kernel, "mean_launch_ms": ms, "dense_gemm_route_ms": dense_ms,
-                "roofline": {"bound": "mfma", "achieved": tf, "peak": MFMA_F32_PEAK_TFLOPS, "unit": "TFLOP/s",
-                             "frac": tf / MFMA_F32_PEAK_TFLOPS, "flops_per_launch": flops},
+                "roofline": {"bound": "mfma", "achieved": tf, "peak": MFMA_SPLIT_PEAK_TFLOPS, "unit": "TFLOP/s",
+                             "frac": tf / MFMA_SPLIT_PEAK_TFLOPS, "flops_per_launch": flops},
                 "algorithmic_bytes": nbytes, "hbm_frac": nbytes / (ms * 1e-3) / 1e9 / HBM_PEAK_GBS}
     return {"workload": "cfg4 MACE message linear (interaction 2): per-degree path blocks 4/6/7/6 x C128 -> C128, "
                         "2,048 atoms, fp32",
@@ -911,7 +914,8 @@ def _bench_radial(device):
 def _mace_floor(edges: int, atoms: int, training: bool):
     """Lower bound on the device time of one cfg-4 step: each modelled piece of work at its own
     roofline (unique bytes at 8 TB/s for the HBM-bound message kernels, useful FLOPs at
-    157.3 TFLOP/s for the GEMMs, the MFMA message linear and the VALU contraction), summed; the
+    157.3 TFLOP/s for the fp32 GEMMs, the radial hidden layers and the VALU contraction, at 417 for
+    the split-bf16 products: the radial network's last layer and the message linear), summed; the
     elementwise glue and the design traffic (bond rows, dxe, gathers beyond the first) count zero.
     Per interaction (input degree 0 then 3; 4 / 23 paths, 16 / 99 message output rows):
     inference = forward + force backward (message VJP, radial-MLP and linear input adjoints, the
@@ -923,12 +927,12 @@ def _mace_floor(edges: int, atoms: int, training: bool):
     e, n, c, s = edges, atoms, 128, 10
     terms = {}
 
-    def add(name, nbytes=0.0, flops=0.0):
-        terms[name] = terms.get(name, 0.0) + max(nbytes / (HBM_PEAK_GBS * 1e9),
-                                                 flops / (MFMA_F32_PEAK_TFLOPS * 1e12)) * 1e3
+    def add(name, nbytes=0.0, flops=0.0, peak=MFMA_F32_PEAK_TFLOPS):
+        terms[name] = terms.get(name, 0.0) + max(nbytes / (HBM_PEAK_GBS * 1e9), flops / (peak * 1e12)) * 1e3
     for lin, npath, noc, target in ((0, 4, 16, 3), (3, 23, 99, 0)):
         nx = (lin + 1) ** 2
-        radial = 2 * e * (8 * 64 + 2 * 64 * 64 + 64 * npath * c)         # radial MLP forward
+        hidden = 2 * e * (8 * 64 + 2 * 64 * 64)                          # radial MLP forward
+        last = 2 * e * 64 * npath * c                                     # its last layer: the gates
         fwd_b = e * (4 * npath * c + 64 + 8) + n * 4 * c * (nx + noc)
         vjp_b = e * (8 * npath * c + 64 + 64 + 8) + n * 4 * c * (2 * nx + noc)
         lin_f = 2 * n * c * c * noc                                       # message linear
@@ -936,16 +940,18 @@ def _mace_floor(edges: int, atoms: int, training: bool):
         sc = sc_flops.flop_counts(3, target, 3)
         sc_f = (sc["forward"] + sc["vjp"]) * n * c
         add("message kernels", nbytes=fwd_b + vjp_b)
-        add("radial MLP", flops=2 * radial)
-        add("message linear", flops=2 * lin_f)
+        add("radial MLP", flops=2 * hidden)
+        add("radial MLP", flops=2 * last, peak=MFMA_SPLIT_PEAK_TFLOPS)
+        add("message linear", flops=2 * lin_f, peak=MFMA_SPLIT_PEAK_TFLOPS)
         add("channel linears", flops=2 * chan_f)
         add("symmetric contraction", flops=sc_f)
         if training:
             tfwd_b = e * (8 * npath * c + 128 + 8) + n * 4 * c * (2 * nx + noc)
             tvjp_b = e * (12 * npath * c + 128 + 64 + 8) + n * 4 * c * (3 * nx + noc)
             add("message kernels", nbytes=vjp_b + tfwd_b + tvjp_b)
-            add("radial MLP", flops=4 * radial)
-            add("message linear", flops=4 * lin_f)
+            add("radial MLP", flops=4 * hidden)
+            add("radial MLP", flops=4 * last, peak=MFMA_SPLIT_PEAK_TFLOPS)
+            add("message linear", flops=4 * lin_f, peak=MFMA_SPLIT_PEAK_TFLOPS)
             add("channel linears", flops=4 * chan_f)
             add("symmetric contraction", flops=2 * sc_f)
     return {"terms_ms": terms, "t_min_ms": sum(terms.values())}

@@ -704,7 +704,9 @@ int launch(const ictc_degree_linear_desc* desc, const float* in, const float* co
 // MFMA; error against float64 1.7e-7, 4.4e-7 there.
 enum WgLayout { kWgIrMul = 0, kWgMulIr = 1 };
 constexpr int kWgMinRows = 256;   // shortest range (8 chunks)
-constexpr int kWgBlocksPerCu = 3;  // 36,864 B of LDS and 80 VGPRs
+// 36,864 B of LDS and 80 VGPRs (six waves per SIMD), which spills 4 VGPRs in the ir_mul layout, 2 in mul_ir
+// (20 and 12 bytes of scratch per lane)
+constexpr int kWgBlocksPerCu = 3;
 constexpr int kWgO = 128, kWgJ = 64;
 constexpr int kWgWaves = 8;   // waves per block: 32 o x 32 j each
 

@@ -207,7 +207,8 @@ tp_forward_kernel(const float* __restrict__ x, const float* __restrict__ y,
 // Outputs whose pointer is null get an empty buffer descriptor: their stores are
 // dropped by the hardware range check, so the instance body has no branches.
 // NV = 2 asks for three waves per SIMD (168 registers; the <3,3,3,2> instance needs 170 without
-// the bound and measured 2.07 ms at two waves per SIMD, 2.04 ms at three).
+// the bound and measured 2.07 ms at two waves per SIMD, 2.04 ms at three; with the path weight it
+// spills 2 of its 168, 12 bytes of scratch per lane).
 template <int LIN, int LE, int LOUT, int NV, bool WEIGHTED>
 __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(NV == 2 ? 3 : 1)))
 tp_backward_kernel(const float* __restrict__ x, const float* __restrict__ y,

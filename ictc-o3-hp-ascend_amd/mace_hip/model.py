@@ -89,7 +89,7 @@ class ChannelLinear(nn.Module):
 
     def to_ir_mul(self, x: torch.Tensor) -> torch.Tensor:
         """mul_ir [N, C(L+1)^2] -> ir_mul [N, sum_l (2l+1) C]: out[n, m, o] = sum_c W[o,c] x[n,c,m],
-        one fp32-MFMA launch over every degree (the message linear's adjoint kernel with the
+        one matrix-core launch over every degree (the message linear's adjoint kernel with the
         weights transposed; the layout change folded into its tile loads and stores)."""
         width = self.channels * (self.lmax + 1) ** 2
         if x.shape[1] != width:
@@ -100,7 +100,7 @@ class ChannelLinear(nn.Module):
 class MessageLinear(nn.Module):
     """PathPreservingLinearSO3 (pure_cartesian_ictd_fix.py:629-661) reading the packed ir_mul
     message (per degree: [count_l paths][2l+1][C]) and writing mul_ir [N, C(L+1)^2]: one
-    fp32-MFMA launch over every degree (degree_linear), the layout changes folded into its tile
+    matrix-core launch over every degree (degree_linear), the layout changes folded into its tile
     loads and stores and the 1/avg_num_neighbors scale passed as its alpha."""
 
     def __init__(self, counts: Dict[int, int], channels: int, lmax: int):
@@ -151,7 +151,7 @@ class IrrepsLinear(nn.Module):
         self.plan = DegreeLinearPlan([1] * (lmax + 1), channels, channels)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        """One fp32-MFMA launch over every degree, mul_ir in and out, 1/sqrt(C) as its alpha."""
+        """One matrix-core launch over every degree, mul_ir in and out, 1/sqrt(C) as its alpha."""
         return degree_linear_mul_ir(x, list(self.weights), self.plan, 1.0 / math.sqrt(self.channels))
 
 

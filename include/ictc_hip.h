@@ -587,8 +587,8 @@ int ictc_hip_radial_mlp(int mode, const float* feats, const float* w1, const flo
                         int num_basis, int64_t edges, hipStream_t stream);
 
 /*
- * Per-degree channel linear on fp32 MFMA (v_mfma_f32_16x16x4_f32), for the path-preserving
- * message linear of the MACE interaction (reference
+ * Per-degree channel linear on the matrix cores (bf16 with fp32 operands in three parts where
+ * the call gives every CU a block, else v_mfma_f32_16x16x4_f32), for the path-preserving message linear of the MACE interaction (reference
  * mace_ictc/models/pure_cartesian_ictd_fix.py:629-661; native route ictc_o3/ascendc/linear.py:
  * 12-136), reading the message kernels' packed output directly.  For degree l (d = 2l + 1):
  *   x [nodes, sum_l counts[l] d C]: per node and degree, counts[l] path blocks of [d][C]

@@ -15,7 +15,8 @@
 // concatenation, the 1/avg_num_neighbors scale as alpha).
 //
 // Calls that give every CU a block run on the bf16 matrix cores with fp32 operands in three parts (the split
-// kernels below), the weight gradient always; smaller calls on fp32 MFMA, in more and smaller blocks:
+// kernels below; `launch` has the lines), the weight gradient always; smaller calls, and short products of up
+// to 64 columns, on fp32 MFMA, in more and smaller blocks:
 //
 // Tiling: a 256-thread block computes a 64-row x 64-column output tile of one degree (grid.z);
 // K is walked in chunks of 32 staged through LDS, then each wave runs v_mfma_f32_16x16x4_f32 over
@@ -651,9 +652,15 @@ int launch(const ictc_degree_linear_desc* desc, const float* in, const float* co
   if (vec && MODE == kInputGrad && max_cols > 64 &&
       (desc->out_channels == 64 || desc->out_channels == 96 || desc->out_channels == 128) &&
       128 * a.xwidth * 4 < 0x40000000) {
-    // the register-resident rows where its 128-row blocks give every CU one
+    // The register-resident rows where its 128-row blocks give every CU one.  A single degree (d = 1: every
+    // load and store of the fp32 kernel is contiguous) has to fill the chip a few times over, counted in blocks
+    // of one 64-column chunk.  us on either side of the line, fp32 in brackets, O = 128: one path block, 49,152
+    // nodes 28.1 (27.2), 65,536 30.5 (34.1); four, 12,288 nodes 29.2 (27.0), 16,384 30.0 (33.8); O = 64: four,
+    // 16,384 nodes 15.6 (14.8), 20,480 17.5 (19.0).
     const LinearSplit sp = input_grad_split(a, degrees);
-    if (sp.block0[degrees] >= compute_units() && sp.block0[degrees] <= 0x7fffffff) {
+    const int64_t single = ((a.g[0].rows + 127) / 128) * ((a.g[0].k + 63) / 64);
+    const bool fills = degrees > 1 || single > (desc->out_channels > 64 ? 3 : 2) * static_cast<int64_t>(compute_units());
+    if (fills && sp.block0[degrees] >= compute_units() && sp.block0[degrees] <= 0x7fffffff) {
       const dim3 igrid(static_cast<unsigned>(sp.block0[degrees]));
       if (desc->out_channels == 64)
         hipLaunchKernelGGL(degree_linear_input_grad_kernel<4>, igrid, dim3(256), 0, stream, in, out, a, sp);
@@ -665,12 +672,22 @@ int launch(const ictc_degree_linear_desc* desc, const float* in, const float* co
     }
   }
   if constexpr (MODE != kInputGrad) {
-    // split-bf16 blocks (two per CU) where they give every CU one: fewer, larger blocks than the fp32
-    // kernel's, which keeps the smaller calls
+    // Split-bf16 blocks (two per CU) where they give every CU one: fewer, larger blocks than the fp32
+    // kernel's, which keeps the smaller calls.  A 64-column block stages as many rows as a 128-column one for
+    // half the products, so that its K has to be long: C = O = 64, lmax 3, 4,096 nodes, one path block (K = 64)
+    // 14.8 us (fp32 13.6), two (K = 128) 18.5 (18.6), four 27.0 (27.3), and at 2,048 nodes two 11.4 (15.0), four
+    // 16.5 (24.4); C = O = 32, 4,096 nodes, one 10.2 (8.3), three (K = 96) 14.1 (13.2), and at 2,048 nodes three
+    // 8.8 (11.3).  A single degree (d = 1: contiguous in the fp32 kernel too) starts at 5/4 of the CUs: 128 x
+    // 128, 16,384 nodes 10.5 (9.2), 20,480 12.1 (12.2), 32,768 14.0 (16.5).
     const int stn = max_cols > 64 ? 128 : 64;
-    int64_t blocks = 0;
-    for (int l = 0; l < degrees; ++l) blocks += ((a.g[l].rows + kTile - 1) / kTile) * ((a.out_channels + stn - 1) / stn);
-    if (vec && blocks >= compute_units()) {
+    int64_t blocks = 0, rows = 0, steps = 0;
+    for (int l = 0; l < degrees; ++l) {
+      blocks += ((a.g[l].rows + kTile - 1) / kTile) * ((a.out_channels + stn - 1) / stn);
+      rows += a.g[l].k > 0 ? a.g[l].rows : 0;
+      steps += a.g[l].rows * a.g[l].k;
+    }
+    const bool deep = stn == 128 || steps >= 96 * rows;
+    if (vec && deep && 4 * blocks >= (degrees > 1 ? 4 : 5) * static_cast<int64_t>(compute_units())) {
       const dim3 sgrid(static_cast<unsigned>(row_tiles), static_cast<unsigned>((max_cols + stn - 1) / stn),
                        static_cast<unsigned>(degrees));
       if (stn == 128)

@@ -1,5 +1,5 @@
-"""The per-degree linear's split-bf16 kernels at sizes that take them (a block for every CU): forward, input
-adjoint, mul_ir maps and weight adjoint against float64, with rows that do not fill a tile, column
+"""The per-degree linear's split-bf16 kernels at sizes that take them (a block for every CU) and on both sides
+of the dispatch's lines: forward, input adjoint, mul_ir maps and weight adjoint against float64, with rows that do not fill a tile, column
 chunks that cross a path block (C = 96), a degree without path blocks, outputs wider than a tile, and
 non-finite values as in float32.
 
@@ -17,7 +17,10 @@ from ictc_o3.backends.hip import degree_linear as D  # noqa: E402
 
 DEV = torch.device("cuda", 0)
 CASES = [((4, 6, 7, 6), 128, 128, 1021), ((1, 2), 96, 96, 5001), ((3, 0, 2), 64, 64, 2503), ((2, 3, 1), 32, 160, 2050),
-         ((2, 1), 64, 96, 4100), ((1,), 64, 64, 20003)]
+         ((2, 1), 64, 96, 4100), ((1,), 64, 64, 20003),
+         # beside the lines of the dispatch: a single degree's blocks, K of a 64-column tile
+         ((4,), 64, 64, 20480), ((4,), 64, 64, 20416), ((1,), 128, 128, 49217), ((1,), 128, 128, 49152),
+         ((1, 1, 2), 64, 64, 2100), ((2, 1, 1), 64, 64, 2100)]
 
 
 def _data(counts, c, o, nodes):
@@ -51,7 +54,8 @@ def test_products_match_float64(counts, c, o, nodes):
     assert torch.equal(D._input_grad_raw(plan, gy, ws, 0.5), 0.5 * gx)
 
 
-@pytest.mark.parametrize("c,o,lmax,nodes", [(128, 128, 3, 1100), (96, 64, 2, 2100), (64, 128, 1, 4200), (32, 32, 3, 1500)])
+@pytest.mark.parametrize("c,o,lmax,nodes", [(128, 128, 3, 1100), (96, 64, 2, 2100), (64, 128, 1, 4200), (32, 32, 3, 1500),
+                                              (128, 64, 2, 2100)])
 def test_mul_ir_maps_match_float64(c, o, lmax, nodes):
     plan, _, gy, ws = _data((1,) * (lmax + 1), c, o, nodes)
     x = torch.randn(nodes, c * (lmax + 1) ** 2, device=DEV)

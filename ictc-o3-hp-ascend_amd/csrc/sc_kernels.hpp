@@ -138,12 +138,18 @@ sc_kernel(const float* __restrict__ x, const float* __restrict__ t, const int64_
 // per CU); wider plans would leave the CUs with one or two waves and keep the features.
 constexpr int kScWgColumns = 96;
 
-// Node ranges per chunk: as many waves as fit the chip (by their LDS), four nodes each at least.
+// Node ranges per chunk: as many waves as fit the chip (by their LDS), `least` nodes each at least: a wave's nodes
+// are one after the other, a range is one more slot for the sum, which adds a species' slots one after the
+// other.  Forward and both gradients with 1, 2 and 4 nodes at least, us, C = 64:
+//   lmax 3 -> 0e+1o, correlation 3   100 nodes 57 64 73, 300 61 65 74, 1,000 79 78 80, 2,000 89 90 94
+//   lmax 1, correlation 3            100 nodes 32 33 34, 300 34 34 34, 1,000 42 38 36, 2,000 55 43 40
+// (writing the features and multiplying them with one-hot rows: 61, 65, 79 at 100, 300, 1,000 nodes of the first)
 inline int64_t sc_wg_ranges(int ktot, int C, int64_t nodes) {
   const int64_t nchunks = (C + kWave - 1) / kWave;
   int64_t per_cu = (160 * 1024) / (static_cast<int64_t>(ktot) * kWave * 4);
   per_cu = per_cu < 16 ? per_cu : 16;
-  const int64_t want = (per_cu * compute_units() + nchunks - 1) / nchunks, most = (nodes + 3) / 4;
+  const int64_t least = nodes <= 300 ? 1 : nodes <= 1200 ? 2 : 4;
+  const int64_t want = (per_cu * compute_units() + nchunks - 1) / nchunks, most = (nodes + least - 1) / least;
   const int64_t r = want < most ? want : most;
   return r < 1 ? 1 : r;
 }

@@ -32,6 +32,7 @@ def _features(plan, x, species, go, t):
 
 @pytest.mark.parametrize("plan_args,channels,elements,nodes", [
     ((3, 1, 3), 128, 10, 1543), ((3, 0, 3), 64, 3, 257), ((2, 2, 3), 24, 89, 300), ((1, 1, 2), 130, 1, 5000),
+    ((1, 1, 3), 64, 4, 301), ((2, 0, 3), 32, 9, 1200), ((2, 0, 3), 32, 9, 1201),    # the shortest ranges' lines
     ((0, 0, 1), 1, 2, 1), ((3, 3, 2), 96, 5, 33), ((3, 1, 3), 64, 7, 40000)])
 @pytest.mark.parametrize("tangent", [False, True])
 def test_weight_gradient_matches_summed_features(plan_args, channels, elements, nodes, tangent):

@@ -6,15 +6,21 @@ it first and keeps its library routes for every other shape.
 
 The lines between the routes (MI355X, us per call in a replayed graph, the library's time in brackets):
 
-* forward from 2,048 rows and 3.5 M results: a block has its rows to load and split before its first
+* forward from 2,048 rows and 6 M results: a block has its rows to load and split before its first
   product, so that a small launch takes 6 us whatever its size: 6.0 (2.7) at 2,048 x 128, 6.9 (5.8) at 5,500 x
-  352, 7.0 (6.2) at 3,500 x 704, 6.9 (5.7) at 20,000 x 128; from the line on 7.6 (8.6) at 7,000 x 512, 10.0 (12.3)
-  at 2,048 x 2,944, 11.5 (14.7) at 20,000 x 352, 288 (408) at 105,634 x 2,944, and at worst 9.8 (9.2) at 20,000 x 256;
+  352, 7.0 (6.2) at 3,500 x 704, 6.9 (5.7) at 20,000 x 128.  Between 3.5 and 6 M the two are close alone, 10.3 (11.1)
+  at 16,000 x 288, 10.0 (8.9) at 40,000 x 128, but between other kernels the library is ahead (that size with its radial
+  kernels and adjoints 48.6, 44.5); from the line on 9.8 (10.3) at 16,000 x 384, 10.0 (12.3) at 2,048 x 2,944, 16.9 (18.0) at
+  28,000 x 352, 288 (408) at 105,634 x 2,944;
 * input adjoint from 50,000 rows: a block takes 128 rows and a fixed 1.1 us per 32 columns, so fewer
   rows leave CUs idle: 105 (88) at 8,192 x 2,944, 120 (108) at 32,768 x 2,944, 176 (225) at 50,000 x 2,944, 40 (40) at
   65,000 x 512, 81 (94) at 105,634 x 704, 311 (373) at 105,634 x 2,944.  A second round of blocks begins above
   131,072 rows and costs 36 us at 2,944 columns, less than the lead: 365 (466) at 131,072, 401 (480) at 131,200,
   418 (481) at 140,000, 599 (714) at 211,000; 59 (60) at 131,200 x 352, 28 (28) at 140,000 x 128;
+* both of these from rows of whole 64-byte lines: the kernels stream the [E, N] rows past the caches, which the lines
+  that two rows share do not bear.  At 105,000 rows forward 34 (28) at 132 columns, 44 (36) at 200, 54 (45) at 264, 114
+  (84) at 552, but 22 (26) at 144, 27 (32) at 176, 52 (60) at 400, 66 (75) at 528; input adjoint 44 (42) at 264, 50 (46) at
+  300, 83 (74) at 552, but 44 (45) at 352, 57 (58) at 480;
 * weight adjoint from 4,096 rows, or 2,048 from 640 columns: 15 (11) at 2,048 x 128, 15 (12) at 2,048 x 512, 17 (16)
   at 4,000 x 512; 16 (18) at 2,048 x 704, 17 (33) at 8,000 x 128, 22 (23) at 8,000 x 704, 19 (25) at 16,000 x 128,
   156 (216) at 105,634 x 1,408.
@@ -30,11 +36,12 @@ from ... import _lib
 WIDTH = 64
 MIN_OUTER = 128            # narrower outer sides stay on the library (its 64 x 64 products take one tile)
 FORWARD_ROWS = 2048
-FORWARD_RESULTS = 3_500_000
+FORWARD_RESULTS = 6_000_000
 INPUT_GRAD_ROWS = 50000
 WEIGHT_GRAD_ROWS = 2048
 WEIGHT_GRAD_NARROW = 640   # narrower outer sides ...
 WEIGHT_GRAD_NARROW_ROWS = 4096   # ... from these rows
+LINE = 16                  # floats of a 64-byte line
 MAX_OUTER = 1 << 20
 MAX_ROW_STRIDE = 1 << 22
 
@@ -42,6 +49,11 @@ MAX_ROW_STRIDE = 1 << 22
 def _rows(t: torch.Tensor, width: int) -> bool:
     """t [R, width] read row by row: unit column stride, rows that do not overlap."""
     return t.stride(1) == 1 and width <= t.stride(0) <= MAX_ROW_STRIDE
+
+
+def _lines(t: torch.Tensor) -> bool:
+    """Rows that start on a 64-byte line."""
+    return t.stride(0) % LINE == 0 and t.data_ptr() % (4 * LINE) == 0
 
 
 def _hidden(t: torch.Tensor) -> bool:
@@ -107,9 +119,10 @@ def product(a: torch.Tensor, b: torch.Tensor, out: Optional[torch.Tensor] = None
         return None
     if a.dtype != torch.float32 or b.dtype != torch.float32:
         return None
-    if forward and _hidden(a) and _weight(b.t()) and (out is None or _rows(out, n)):
+    if (forward and _hidden(a) and _weight(b.t())
+            and (n % LINE == 0 if out is None else _rows(out, n) and _lines(out))):
         return _forward(a, b.t(), out)
-    if (input_grad and _rows(a, k) and a.stride(0) % 4 == 0 and a.data_ptr() % 16 == 0 and _weight(b)
+    if (input_grad and _rows(a, k) and _lines(a) and _weight(b)
             and (out is None or (out.stride(0) == WIDTH and out.stride(1) == 1))):
         return _input_grad(a, b, out)
     if weight_grad and n == WIDTH and _rows(a.t(), m) and b.stride(1) == 1 and b.stride(0) == WIDTH:

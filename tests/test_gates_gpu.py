@@ -83,12 +83,17 @@ def test_non_finite_and_huge_values_as_in_float32():
 def test_rule_takes_the_three_forms_and_leaves_the_rest(monkeypatch):
     for name in ("FORWARD_ROWS", "FORWARD_RESULTS", "INPUT_GRAD_ROWS", "WEIGHT_GRAD_ROWS", "WEIGHT_GRAD_NARROW_ROWS"):
         monkeypatch.setattr(G, name, 256)
-    h, w, g = _inputs(300, 132)
+    h, w, g = _inputs(300, 144)
     for a, b in ((h, w.t()), (h, w.t().contiguous()), (g, w), (g, w.t().contiguous().t()), (g.t(), h), (h.t(), g)):
         got = G.product(a, b)
         assert got is not None and torch.equal(got, L._product(a, b))
         _close(got, a, b)
-    odd = torch.empty(300 * 132 + 1, device=DEV)[1:].reshape(300, 132).copy_(g)     # not 16-byte aligned
+    odd = torch.empty(300 * 144 + 1, device=DEV)[1:].reshape(300, 144).copy_(g)     # not 16-byte aligned
+    shared = [t[:, :132] for t in (g.reshape(-1)[:300 * 132].reshape(300, 132), g)]   # rows that share lines, and not
+    assert G.product(shared[0], w[:132]) is None and G.product(shared[1], w[:132]) is not None
+    room = torch.empty(300, 160, device=DEV)
+    assert G.product(h, w.t(), room[:, :144]) is not None and G.product(h, w.t(), room[:, 8:152]) is None
+    assert G.product(h, w[:136].t()) is None
     refused = [(odd, w), (h[:, :32], w[:, :32].t()), (h[:100], w.t()), (h, w[:64].t()), (h[::2], w.t()),
                (g[:, :131], w[:131]), (h.expand(300, 64)[:1].expand(300, 64), w.t()), (h.double(), w.double().t())]
     for a, b in refused:
@@ -98,9 +103,9 @@ def test_rule_takes_the_three_forms_and_leaves_the_rest(monkeypatch):
 
 
 @pytest.mark.parametrize("rows,width,forward,weight", [
-    (6835, 512, False, True), (6836, 512, True, True), (2048, 1708, False, True), (2048, 1709, True, True),
+    (11718, 512, False, True), (11719, 512, True, True), (2048, 2928, False, True), (2048, 2944, True, True),
     (2047, 2944, False, False), (27000, 128, False, True), (4095, 636, False, False), (4095, 640, False, True),
-    (4096, 128, False, True)])
+    (4096, 128, False, True), (46000, 132, False, True)])
 def test_lines_of_the_rule(rows, width, forward, weight):
     h, w, g = _inputs(rows, width)
     for a, b, taken in ((h, w.t(), forward), (g.t(), h, weight), (h.t(), g, weight), (g, w, False)):

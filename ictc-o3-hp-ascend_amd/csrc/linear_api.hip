@@ -652,14 +652,20 @@ int launch(const ictc_degree_linear_desc* desc, const float* in, const float* co
   if (vec && MODE == kInputGrad && max_cols > 64 &&
       (desc->out_channels == 64 || desc->out_channels == 96 || desc->out_channels == 128) &&
       128 * a.xwidth * 4 < 0x40000000) {
-    // The register-resident rows where its 128-row blocks give every CU one.  A single degree (d = 1: every
-    // load and store of the fp32 kernel is contiguous) has to fill the chip a few times over, counted in blocks
-    // of one 64-column chunk.  us on either side of the line, fp32 in brackets, O = 128: one path block, 49,152
-    // nodes 28.1 (27.2), 65,536 30.5 (34.1); four, 12,288 nodes 29.2 (27.0), 16,384 30.0 (33.8); O = 64: four,
-    // 16,384 nodes 15.6 (14.8), 20,480 17.5 (19.0).
+    // The register-resident rows where its 128-row blocks give every CU one.  Counted in blocks of one
+    // 64-column chunk, a single degree (d = 1: every load and store of the fp32 kernel is contiguous) has to
+    // fill the chip a few times over, and up to 128 columns of more than 64 outputs whole rounds of one or two
+    // blocks per CU: a CU's second block costs 6 us of 16.  us on either side of the lines, fp32 in brackets:
+    // single degree, O = 128, one path block, 49,152 nodes 28.1 (27.2), 65,536 30.5 (34.1); four, 12,288 nodes
+    // 29.2 (27.0), 16,384 30.0 (33.8); O = 64, four, 16,384 nodes 15.6 (14.8), 20,480 17.5 (19.0); several degrees,
+    // O = 128, one path block: 256 blocks 15.8 (17.6, lmax 3), 260 21.0 (17.1, lmax 2), 320 20.9 (18.0, lmax 3),
+    // 384 22.6 (24.1, lmax 2), 21.5 (18.3, lmax 3), 512 23.2 (29.8, lmax 3).
     const LinearSplit sp = input_grad_split(a, degrees);
-    const int64_t single = ((a.g[0].rows + 127) / 128) * ((a.g[0].k + 63) / 64);
-    const bool fills = degrees > 1 || single > (desc->out_channels > 64 ? 3 : 2) * static_cast<int64_t>(compute_units());
+    const int64_t cus = compute_units();
+    int64_t chunked = 0;
+    for (int l = 0; l < degrees; ++l) chunked += (a.g[l].rows + 127) / 128 * ((a.g[l].k + 63) / 64);
+    const bool fills = degrees == 1 ? chunked > (desc->out_channels > 64 ? 3 : 2) * cus
+                                    : max_cols > 128 || desc->out_channels == 64 || chunked <= cus || chunked >= 2 * cus;
     if (fills && sp.block0[degrees] >= compute_units() && sp.block0[degrees] <= 0x7fffffff) {
       const dim3 igrid(static_cast<unsigned>(sp.block0[degrees]));
       if (desc->out_channels == 64)

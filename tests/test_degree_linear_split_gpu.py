@@ -20,7 +20,8 @@ CASES = [((4, 6, 7, 6), 128, 128, 1021), ((1, 2), 96, 96, 5001), ((3, 0, 2), 64,
          ((2, 1), 64, 96, 4100), ((1,), 64, 64, 20003),
          # beside the lines of the dispatch: a single degree's blocks, K of a 64-column tile
          ((4,), 64, 64, 20480), ((4,), 64, 64, 20416), ((1,), 128, 128, 49217), ((1,), 128, 128, 49152),
-         ((1, 1, 2), 64, 64, 2100), ((2, 1, 1), 64, 64, 2100)]
+         ((1, 1, 2), 64, 64, 2100), ((2, 1, 1), 64, 64, 2100),
+         ((1, 1, 1, 1), 128, 128, 1024), ((1, 1, 1), 96, 96, 2048), ((1, 1, 1, 1), 96, 96, 2048)]
 
 
 def _data(counts, c, o, nodes):

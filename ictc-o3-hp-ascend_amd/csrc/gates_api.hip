@@ -4,10 +4,10 @@
 // (split_bf16.hpp).  E is edge-sized (1e3 .. 1e6), so each product moves one [E, N] fp32 tensor
 // (1.24 GB at E = 105,634, N = 2,944) and should take the time of that stream.
 //
-// Measured at E = 105,634, N = 2,944 (rocBLAS / hipBLASLt fp32 before): gates 265 (385) us = 4.7 TB/s
-// written, input adjoint 300 (353) us, weight adjoint 280 (620: split products and a remainder) us =
-// 5.1 TB/s read; back to back, at the clock the chip then holds, 330 (520), 336 (395), 295 (515) us.  The
-// six part products would take 95 us at the matrix cores' peak (busy 48 / 40 / 49 % of the time).
+// Measured at E = 105,634, N = 2,944, each product by itself in a replayed graph (rocBLAS / hipBLASLt fp32 before):
+// gates 288 (408) us = 4.3 TB/s written, input adjoint 311 (373) us = 4.0 TB/s read, weight adjoint 293 (515: split
+// products and a remainder) us = 4.3 TB/s read.  The six part products would take 95 us at the matrix cores' peak;
+// one after the other in a training pass the matrix cores are busy 41, 40 and 47 % of the time.
 // Errors against float64 (2-norm): 1.1e-7 (1.4e-7), 3.3e-7 (9.7e-7), 1.1e-6 (3.1e-6).
 //
 // Every kernel: 256 threads, v_mfma_f32_32x32x16_bf16.  The operand that all edges share (W, or h for
@@ -198,7 +198,8 @@ struct StepTile {
 __device__ __forceinline__ int stage_slot(int r, int p) { return r * 8 + (p ^ (r & 7)); }
 
 // Four blocks per CU (128 VGPRs, 40 KB of LDS): the 826 blocks of E = 105,634 are then resident at once
-// (at three per CU a second round of 58 blocks doubled the time).
+// (at three per CU a second round of 58 blocks doubled the time).  Above E = 131,072 a second round begins here: 365
+// us at 131,072, 401 at 131,200 (library 466, 480).
 __global__ void __launch_bounds__(kGThreads, 4)
 gates_input_grad_kernel(const float* __restrict__ g, int64_t ldg, const float* __restrict__ w, int64_t wsn, int64_t wsk,
                         float* __restrict__ out, int64_t E, int N) {

@@ -296,7 +296,7 @@ degree_linear_kernel(const float* __restrict__ in, float* __restrict__ out, cons
 // matrix instructions (two LDS buffers, one barrier per chunk).  Wave w computes rows 32 (w % 2) ..
 // and columns (TN / 2) (w / 2) ..  The small part products have accumulators of their own.
 // Bound by the staging between barriers at two blocks per CU.  2048 nodes, C = O = 128, counts (4, 6, 7, 6)
-// (19.9 GFLOP over forward and both adjoints): 51 us, on fp32 MFMA 75 us; error against float64 1.6e-7, 5.0e-7
+// (19.9 GFLOP over forward and both adjoints): 52 us, on fp32 MFMA 75 us; error against float64 1.6e-7, 5.0e-7
 // there.  One LDS buffer with two barriers per chunk (three blocks per CU): 61 us.
 constexpr int kSpRows = kTile + 2;       // units per octet row: staggers the staging writes' banks
 
@@ -443,9 +443,9 @@ degree_linear_split_kernel(const float* __restrict__ in, float* __restrict__ out
 // flight), its columns in the order even, odd so that a lane owns two neighbouring ones and stores
 // them together (256 contiguous bytes of two rows per instruction).  LinearSplit lists the launch's blocks:
 // 128 rows of one degree times `chunks` column chunks.
-// 2048 nodes, C = O = 128, counts (4, 6, 7, 6): 56 us, on fp32 MFMA 84 us (the six part products take about 29,
-// the 104 MB of gx 15; the rest is the first loads and the last partly filled round of blocks); error
-// against float64 1.6e-7, 2.0e-7 there.
+// 2048 nodes, C = O = 128, counts (4, 6, 7, 6): 54 us, on fp32 MFMA 84 us (the six part products take 16 at the
+// matrix cores' peak, the 104 MB of gx 13 at HBM's; the rest is the first loads and the last partly filled
+// round of blocks); error against float64 1.6e-7, 2.0e-7 there.
 struct LinearSplit {
   int64_t block0[ICTC_LINEAR_MAX_DEGREES + 1];   // first block of each degree
   int splits[ICTC_LINEAR_MAX_DEGREES];           // column splits of a degree
@@ -723,7 +723,7 @@ int launch(const ictc_degree_linear_desc* desc, const float* in, const float* co
 // flight during the current chunk's matrix instructions (one LDS buffer, two barriers per chunk).  The
 // partials go to the workspace; a second kernel sums the ranges in order and scales by alpha (fixed order:
 // bit-identical run to run).  Rows past the end read zeros from the buffer range check (their offsets lie
-// past the tensors).  2048 nodes, C = O = 128, counts (4, 6, 7, 6): 82 us with the sum, 101 us with fp32
+// past the tensors).  2048 nodes, C = O = 128, counts (4, 6, 7, 6): 80 us with the sum, 101 us with fp32
 // MFMA; error against float64 1.7e-7, 4.4e-7 there.
 enum WgLayout { kWgIrMul = 0, kWgMulIr = 1 };
 constexpr int kWgMinRows = 256;   // shortest range (8 chunks)

@@ -50,6 +50,8 @@ class TensorProductPlan:
     kernels; a degree of 4 to 6 runs the degree-generic ones (``generic``), which have no
     fused message tangent kernels."""
 
+    _weight_capacity: Optional[int] = None   # of the class: plans saved before there was one have none
+
     def __init__(self, paths: Sequence[Tuple[int, int, int]], channels: int, input_lmax: int,
                  edge_lmax: int, lmax: Optional[int] = None):
         paths = [tuple(int(v) for v in p) for p in paths]
@@ -82,7 +84,6 @@ class TensorProductPlan:
             desc.out_offset[s] = offsets[s]
             desc.scale[s] = self.plan.scales[index[p]] if p in index else 0.0
         self.desc = desc
-        self._weight_capacity = None
         self.num_paths = len(paths)
         self.full_paths = full
         self.is_full = paths == full

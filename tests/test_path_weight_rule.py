@@ -1,6 +1,8 @@
 """What the tensor product's path weight must be for the kernels to fold it into the gates
 (``gates_and_weight``): every other weight takes the separate product ``gates * weight``, as before the
 kernels took one.  CPU only (no kernel runs)."""
+import copy
+
 import pytest
 import torch
 
@@ -85,3 +87,11 @@ def test_a_forward_mode_tangent_is_not_dropped(monkeypatch):
         x, y = torch.randn(ROWS, 9 * C), torch.randn(ROWS, 9)
         with pytest.raises(RuntimeError, match="jvp"):
             T.packed_tensor_product(plan, x, y, gates, weight)
+
+
+def test_a_plan_saved_without_a_weight_capacity():
+    """Modules saved whole before plans had the attribute hold plans without it."""
+    _, plan, _ = _owner()
+    want, saved = plan.weight_capacity, copy.copy(plan)
+    saved.__dict__ = {k: v for k, v in plan.__dict__.items() if "capacity" not in k}
+    assert saved.weight_capacity == want > 0

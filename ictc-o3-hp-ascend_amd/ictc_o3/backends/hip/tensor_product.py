@@ -254,7 +254,9 @@ def gates_and_weight(owner, plan: TensorProductPlan, gates: Optional[torch.Tenso
     (every path of a compiled degree set, P*C up to ``weight_capacity``; they read P*C floats, so a weight
     that broadcasts against [P, C] does not go there), which saves a pass over the gates and one
     over their gradients; otherwise it is multiplied into the gates here
-    (``owner.effective_gates``).  Both read the weight on every call and round the same products."""
+    (``owner.effective_gates``).  Both read the weight on every call and round the same products.  Gates that
+    the kernels fold are kept for the backward as they are, like the features: a caller that writes into
+    them before the backward passes a copy."""
     w = owner.weight
     if (gates is None or not plan.is_full or plan.full_gate_width > plan.weight_capacity
             or w.shape != (plan.num_paths, plan.channels) or w.device != gates.device

@@ -61,7 +61,7 @@ HARM_LMAX = 6
 WIDE_COMBOS = [(4, 4, 4)]
 INSTANCE_KINDS = {
     "fwd": ("tp_kernels.hpp", "template int launch_forward<{a}, {b}, {c}>(const ictc_tp_desc&, "
-            "const float*, const float*, const float*, const float*, float*, int64_t, hipStream_t);"),
+            "const float*, const float*, const float*, const float*, float*, float*, int64_t, hipStream_t);"),
     "bwd": ("tp_kernels.hpp", "template int launch_backward<{a}, {b}, {c}>(const ictc_tp_desc&, "
             "const float*, const float*, const float*, const float*, const float*, float*, float*, float*, "
             "int64_t, hipStream_t);"),

@@ -8,8 +8,8 @@ namespace ictc {
 // Explicit instantiations live in separate translation units (parallel build).
 #define ICTC_DECLARE(A, B, C)                                                                  \
   extern template int launch_forward<A, B, C>(const ictc_tp_desc&, const float*, const float*,   \
-                                              const float*, const float*, float*, int64_t,      \
-                                              hipStream_t);                                     \
+                                              const float*, const float*, float*, float*,       \
+                                              int64_t, hipStream_t);                            \
   extern template int launch_backward<A, B, C>(const ictc_tp_desc&, const float*, const float*,  \
                                                const float*, const float*, const float*, float*,   \
                                                float*, float*, int64_t, hipStream_t);
@@ -20,8 +20,8 @@ namespace ictc {
 // degree-generic kernels.
 #define ICTC_DECLARE(A, B, C)                                                                  \
   extern template int launch_forward<A, B, C>(const ictc_tp_desc&, const float*, const float*,   \
-                                              const float*, const float*, float*, int64_t,      \
-                                              hipStream_t);                                     \
+                                              const float*, const float*, float*, float*,       \
+                                              int64_t, hipStream_t);                            \
   extern template int launch_backward<A, B, C>(const ictc_tp_desc&, const float*, const float*,  \
                                                const float*, const float*, const float*, float*,   \
                                                float*, float*, int64_t, hipStream_t);
@@ -99,7 +99,7 @@ const char* ictc_hip_status_string(int status) {
   }
 }
 
-int ictc_hip_abi_version(void) { return 25; }
+int ictc_hip_abi_version(void) { return 26; }
 
 int ictc_hip_tp_slot_count(int input_lmax, int edge_lmax, int output_lmax) {
   constexpr int L = ictc::kGenericMaxL;
@@ -118,8 +118,8 @@ int ictc_hip_tp_weight_capacity(const ictc_tp_desc* desc) {
 }
 
 int ictc_hip_tp_forward_weighted(const ictc_tp_desc* desc, const float* features, const float* harmonics,
-                                 const float* gates, const float* path_weight, float* out, int64_t rows,
-                                 hipStream_t stream) {
+                                 const float* gates, const float* path_weight, float* weight_copy, float* out,
+                                 int64_t rows, hipStream_t stream) {
   const int st = ictc::tp_check_desc(desc);
   if (st != ICTC_OK) return st;
   if (rows < 0) return ICTC_ERR_INVALID_ARGUMENT;
@@ -128,17 +128,17 @@ int ictc_hip_tp_forward_weighted(const ictc_tp_desc* desc, const float* features
   if (path_weight && int64_t{desc->num_paths} * desc->channels > ictc_hip_tp_weight_capacity(desc))
     return ICTC_ERR_UNSUPPORTED;
   if (const ictc::FwdLaunch wide = ictc::wide_forward(desc))
-    return wide(*desc, features, harmonics, gates, path_weight, out, rows, stream);
+    return wide(*desc, features, harmonics, gates, path_weight, weight_copy, out, rows, stream);
   if (ictc::generic_degrees(*desc))
     return ictc::generic_tp_forward(*desc, features, harmonics, gates, out, rows, stream);
   const ictc::FwdLaunch fn = ictc::kFwdTable[ictc::table_index(desc)];
   if (fn == nullptr) return ICTC_ERR_UNSUPPORTED;
-  return fn(*desc, features, harmonics, gates, path_weight, out, rows, stream);
+  return fn(*desc, features, harmonics, gates, path_weight, weight_copy, out, rows, stream);
 }
 
 int ictc_hip_tp_forward(const ictc_tp_desc* desc, const float* features, const float* harmonics,
                         const float* gates, float* out, int64_t rows, hipStream_t stream) {
-  return ictc_hip_tp_forward_weighted(desc, features, harmonics, gates, nullptr, out, rows, stream);
+  return ictc_hip_tp_forward_weighted(desc, features, harmonics, gates, nullptr, nullptr, out, rows, stream);
 }
 
 int ictc_hip_tp_backward_weighted(const ictc_tp_desc* desc, const float* features, const float* harmonics,

@@ -117,8 +117,8 @@ __device__ __forceinline__ Vec<NV> path_weight(const float* sW, int at) {
 template <int LIN, int LE, int LOUT, int NV, bool WEIGHTED>
 __global__ void __launch_bounds__(kBlock)
 tp_forward_kernel(const float* __restrict__ x, const float* __restrict__ y,
-                  const float* __restrict__ g, const float* __restrict__ w, float* __restrict__ out,
-                  const ictc_tp_desc d, int64_t rows) {
+                  const float* __restrict__ g, const float* __restrict__ w, float* __restrict__ wcopy,
+                  float* __restrict__ out, const ictc_tp_desc d, int64_t rows) {
   extern __shared__ float sW[];   // WEIGHTED: [P, C]
   using PS = Paths<LIN, LE, LOUT>;
   constexpr int NX = PS::NX, NY = PS::NY, NP = PS::N, NOC = PS::NOC;
@@ -144,6 +144,8 @@ tp_forward_kernel(const float* __restrict__ x, const float* __restrict__ y,
   for (int m = 0; m < NX; ++m) xr0[m] = buf_load<NV>(rx0, vo0 + m * row);
 
   stage_weight<WEIGHTED>(w, sW, NP * C, tid);
+  if (WEIGHTED && wcopy != nullptr && blockIdx.x == 0)   // the weight of this call, for its backward
+    for (int t = tid; t < NP * C; t += kBlock) wcopy[t] = w[t];
   stage_tile<LIN, LE, LOUT, kFwdTile>(y, e0, rows, sY, sM, d, tid);
 
   for (int le = wave; le < kFwdTile; le += kWavesPerBlock) {
@@ -476,8 +478,8 @@ tp_backward_wide_kernel(const float* __restrict__ x, const float* __restrict__ y
 }
 
 // ----------------------------------------------------------------------------- launchers
-// w: the frozen path weight [P, C], or null.
-using FwdLaunch = int (*)(const ictc_tp_desc&, const float*, const float*, const float*, const float*, float*,
+// w: the frozen path weight [P, C], or null; the forward's wcopy: where it is copied to, or null.
+using FwdLaunch = int (*)(const ictc_tp_desc&, const float*, const float*, const float*, const float*, float*, float*,
                           int64_t, hipStream_t);
 using BwdLaunch = int (*)(const ictc_tp_desc&, const float*, const float*, const float*, const float*,
                           const float*, float*, float*, float*, int64_t, hipStream_t);
@@ -485,23 +487,23 @@ using BwdLaunch = int (*)(const ictc_tp_desc&, const float*, const float*, const
 inline int launch_status() { return hipGetLastError() == hipSuccess ? ICTC_OK : ICTC_ERR_LAUNCH; }
 
 template <int LIN, int LE, int LOUT, int NV, bool WEIGHTED>
-int launch_forward_as(const ictc_tp_desc& d, const float* x, const float* y, const float* g, const float* w, float* out,
-                      int64_t rows, hipStream_t stream) {
+int launch_forward_as(const ictc_tp_desc& d, const float* x, const float* y, const float* g, const float* w,
+                      float* wcopy, float* out, int64_t rows, hipStream_t stream) {
   const dim3 grid(static_cast<unsigned>((rows + kFwdTile - 1) / kFwdTile));
   const size_t lds = WEIGHTED ? sizeof(float) * d.num_paths * d.channels : 0;
-  hipLaunchKernelGGL((tp_forward_kernel<LIN, LE, LOUT, NV, WEIGHTED>), grid, dim3(kBlock), lds, stream, x, y, g, w, out,
-                     d, rows);
+  hipLaunchKernelGGL((tp_forward_kernel<LIN, LE, LOUT, NV, WEIGHTED>), grid, dim3(kBlock), lds, stream, x, y, g, w, wcopy,
+                     out, d, rows);
   return launch_status();
 }
 
 template <int LIN, int LE, int LOUT>
-int launch_forward(const ictc_tp_desc& d, const float* x, const float* y, const float* g, const float* w, float* out,
-                   int64_t rows, hipStream_t stream) {
+int launch_forward(const ictc_tp_desc& d, const float* x, const float* y, const float* g, const float* w, float* wcopy,
+                   float* out, int64_t rows, hipStream_t stream) {
   if (d.channels % (2 * kWave) == 0)
-    return w ? launch_forward_as<LIN, LE, LOUT, 2, true>(d, x, y, g, w, out, rows, stream)
-             : launch_forward_as<LIN, LE, LOUT, 2, false>(d, x, y, g, w, out, rows, stream);
-  return w ? launch_forward_as<LIN, LE, LOUT, 1, true>(d, x, y, g, w, out, rows, stream)
-           : launch_forward_as<LIN, LE, LOUT, 1, false>(d, x, y, g, w, out, rows, stream);
+    return w ? launch_forward_as<LIN, LE, LOUT, 2, true>(d, x, y, g, w, wcopy, out, rows, stream)
+             : launch_forward_as<LIN, LE, LOUT, 2, false>(d, x, y, g, w, wcopy, out, rows, stream);
+  return w ? launch_forward_as<LIN, LE, LOUT, 1, true>(d, x, y, g, w, wcopy, out, rows, stream)
+           : launch_forward_as<LIN, LE, LOUT, 1, false>(d, x, y, g, w, wcopy, out, rows, stream);
 }
 
 template <int LIN, int LE, int LOUT, int NV, bool WEIGHTED>

@@ -15,7 +15,7 @@ import torch  # noqa: F401  (must precede CDLL, see module docstring)
 
 MAX_PATHS = 128
 LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "lib", "libictc_hip.so")
-ABI_VERSION = 25
+ABI_VERSION = 26
 
 
 class TpDesc(ctypes.Structure):
@@ -64,7 +64,7 @@ _SIGNATURES = {
     "ictc_hip_tp_backward": (ctypes.c_int, [ctypes.POINTER(TpDesc), _P, _P, _P, _P, _P, _P, _P,
                                             _I64, _P]),
     "ictc_hip_tp_weight_capacity": (ctypes.c_int, [ctypes.POINTER(TpDesc)]),
-    "ictc_hip_tp_forward_weighted": (ctypes.c_int, [ctypes.POINTER(TpDesc)] + [_P] * 5 + [_I64, _P]),
+    "ictc_hip_tp_forward_weighted": (ctypes.c_int, [ctypes.POINTER(TpDesc)] + [_P] * 6 + [_I64, _P]),
     "ictc_hip_tp_backward_weighted": (ctypes.c_int, [ctypes.POINTER(TpDesc)] + [_P] * 8 + [_I64, _P]),
     "ictc_hip_direction_harmonics": (ctypes.c_int, [ctypes.c_int, ctypes.c_int, _P, _P, _P, _P, _P,
                                                     _I64, _P]),

@@ -125,12 +125,13 @@ int ictc_hip_tp_backward(const ictc_tp_desc* desc,
  * by the kernels: out = TP(x, Y, g * w), grad_gates = w * d/d(g * w).  Bit-identical to a separate
  * g * w pass (reference ictc_o3/backends/ascend/packed_tensor_product.py:163-164).  P * C at most
  * ictc_hip_tp_weight_capacity(desc) (0: the degree set does not take a weight, -1: bad descriptor), else
- * ICTC_ERR_UNSUPPORTED.
+ * ICTC_ERR_UNSUPPORTED.  weight_copy (or null), P * C floats apart from path_weight: the forward with a weight
+ * and rows > 0 copies path_weight there, for a backward that must not see later changes of it.
  */
 int ictc_hip_tp_weight_capacity(const ictc_tp_desc *desc);
 int ictc_hip_tp_forward_weighted(const ictc_tp_desc *desc, const float *features, const float *harmonics,
-                                 const float *gates, const float *path_weight, float *out, int64_t rows,
-                                 hipStream_t stream);
+                                 const float *gates, const float *path_weight, float *weight_copy, float *out,
+                                 int64_t rows, hipStream_t stream);
 int ictc_hip_tp_backward_weighted(const ictc_tp_desc *desc, const float *features, const float *harmonics,
                                   const float *gates, const float *path_weight, const float *grad_out,
                                   float *grad_features, float *grad_harmonics, float *grad_gates, int64_t rows,

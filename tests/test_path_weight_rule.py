@@ -52,8 +52,10 @@ def test_the_backward_uses_the_weight_of_its_forward(monkeypatch, change):
     owner, plan, gates = _owner()
     seen = []
 
-    def kernels(plan, x, y, g, w=None):
+    def kernels(plan, x, y, g, w=None, copy=None):
         seen.append(w)
+        if copy is not None:
+            copy.copy_(w)
         return x.new_zeros(ROWS, plan.full_out_width)
 
     def adjoint(plan, need, x, y, g, go, w=None):
@@ -78,7 +80,7 @@ def test_a_forward_mode_tangent_is_not_dropped(monkeypatch):
     tangent, so that the call is refused and not answered as if there were none."""
     import torch.autograd.forward_ad as fwad
     owner, plan, gates = _owner()
-    monkeypatch.setattr(T, "_forward_raw", lambda plan, x, y, g, w=None: x.new_zeros(ROWS, plan.full_out_width))
+    monkeypatch.setattr(T, "_forward_raw", lambda plan, x, y, g, w=None, copy=None: x.new_zeros(ROWS, plan.full_out_width))
     with fwad.dual_level():
         del owner.weight
         owner.weight = fwad.make_dual(torch.ones(owner.num_paths, C), torch.ones(owner.num_paths, C))

@@ -67,6 +67,18 @@ def test_weight_changes_are_seen_and_gates_of_rank_three():
         assert torch.equal(op(x, y, g.reshape(20, op.tp.num_paths, 48)), want)
 
 
+@pytest.mark.parametrize("channels,degree,rows", [(1, 0, 1), (24, 1, 40), (128, 3, 33), (97, 4, 5)])
+def test_the_backward_uses_the_weight_of_its_forward(channels, degree, rows):
+    """The kernel's copy of the weight: gradients as before for a weight that changes after the forward."""
+    op = _op(channels, degree, degree, degree)
+    inputs = _inputs(op, rows)
+    go = torch.randn(rows, op.output_width, device=DEV)
+    want = torch.autograd.grad(op(*inputs), inputs, go)
+    out = op(*inputs)
+    op.tp.weight.data.mul_(3.0)
+    assert all(torch.equal(a, b) for a, b in zip(torch.autograd.grad(out, inputs, go), want))
+
+
 def test_separate_product_where_the_kernels_do_not_take_the_weight():
     op = _op(64, 2, 2, 2)
     x, y, g = _inputs(op, 10)

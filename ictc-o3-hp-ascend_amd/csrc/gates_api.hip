@@ -7,7 +7,7 @@
 // Measured at E = 105,634, N = 2,944, each product by itself in a replayed graph (rocBLAS / hipBLASLt fp32 before):
 // gates 288 (408) us = 4.3 TB/s written, input adjoint 311 (373) us = 4.0 TB/s read, weight adjoint 293 (515: split
 // products and a remainder) us = 4.3 TB/s read.  The six part products would take 95 us at the matrix cores' peak;
-// one after the other in a training pass the matrix cores are busy 41, 40 and 47 % of the time.
+// one after the other in a training pass the matrix cores are busy 41, 39 and 47 % of the time.
 // Errors against float64 (2-norm): 1.1e-7 (1.4e-7), 3.3e-7 (9.7e-7), 1.1e-6 (3.1e-6).
 //
 // Every kernel: 256 threads, v_mfma_f32_32x32x16_bf16.  The operand that all edges share (W, or h for
